@@ -58,8 +58,8 @@ KERNEL_OF = {"scan_u32": "scan_tiles_kernel", "sum_f32": "full_reduce_kernel<", 
              "segmented_short_i32": "seg_short_kernel", "scan_f32_2_30": "scan_tiles_kernel",
              "copy_u32": "copy_tiles_kernel", "dot_f32": "map_reduce_kernel<", "axpy_f32": "vector_tiles_kernel<1",
              "colsum_f32": "cols_tiles_kernel", "colscan_u32": "col_lookback_kernel",
-             "colscan_narrow_u32": "col_narrow_scan_kernel", "segmented_long_i32": "segmented_sum_kernel",
-             "colscan_rowtile_u32": "col_rowtile_lookback_kernel", "colscan_rowtile_wide_u32": "col_rowtile_scan_kernel",
+             "colscan_narrow_u32": "col_strip_kernel", "segmented_long_i32": "segmented_sum_kernel",
+             "colscan_rowtile_u32": "col_rowtile_lookback_kernel", "colscan_rowtile_wide_u32": "col_strip_kernel",
              "colsum_period_f32": "cols_period_kernel", "rows_short_f32": "rows_tile_kernel"}
 
 

@@ -301,11 +301,16 @@ struct ScanArgs {
     uint64_t in_offset;
     int64_t out_line_stride, out_elem_stride;
     uint64_t out_offset;
+    // Column scans keep to the chunked form, whose workspace is small.
+    bool small_workspace = false;
 };
 uint64_t scan_workspace_bytes(const ScanArgs &args);
+// The workspace by which hx_scan_noalloc takes or rejects a scan.
+uint64_t scan_fixed_workspace_bytes(const ScanArgs &args);
 // False for chunked column scans, whose workspace holds chunk totals
 // instead of look-back status words (immediate calls take it from device
-// scratch); true for every other scan.
+// scratch), and for short dense lines, which need none; true for every other
+// scan.
 bool scan_uses_lookback(const ScanArgs &args);
 hx_status launch_scan(const ScanArgs &args, void *ws, uint64_t ws_bytes,
                       LookbackState &st, hipStream_t stream);

@@ -38,13 +38,19 @@ hx_status lookup_noalloc_scratch(void **ptr) {
     return HX_OK;
 }
 
-hx_status launch_scan_noalloc(const ScanArgs &a, void *scratch_ptr, hipStream_t stream) {
-    if (a.lines == 0 || a.len == 0) return HX_OK;
-    const uint64_t bytes = scan_workspace_bytes(a);
-    if (bytes > kNoAllocBytes)
+hx_status launch_scan_noalloc(const ScanArgs &args, void *scratch_ptr, hipStream_t stream) {
+    if (args.lines == 0 || args.len == 0) return HX_OK;
+    const uint64_t needs = scan_fixed_workspace_bytes(args);
+    if (needs > kNoAllocBytes)
         return fail(HX_ERR_DISPATCH_FAILED,
                     "scan needs %llu bytes of workspace; the no-allocation scratch holds %llu "
                     "(use hx_scan or hx_prepare_scan)",
+                    (unsigned long long)needs, (unsigned long long)kNoAllocBytes);
+    ScanArgs a = args;
+    a.small_workspace = scan_workspace_bytes(a) > kNoAllocBytes;
+    const uint64_t bytes = scan_workspace_bytes(a);
+    if (bytes > kNoAllocBytes)
+        return fail(HX_ERR_DISPATCH_FAILED, "scan needs %llu bytes of workspace; the no-allocation scratch holds %llu",
                     (unsigned long long)bytes, (unsigned long long)kNoAllocBytes);
     if (scratch_ptr == nullptr)
         return fail(HX_ERR_DEVICE_UNAVAILABLE, "the no-allocation scratch was not set up for this device");

@@ -994,9 +994,13 @@ void scan_short_lines_kernel(ShortParams p) {
 }
 
 // Column scans: many strided lines whose starts are adjacent in memory
-// (axis-0 scan of a row-major matrix).  From 256 lines up they take the
-// single-pass col_lookback_kernel below; narrower matrices take this chunked
-// reduce-then-scan.  Lanes run across lines -- a wave owns 64*V adjacent
+// (axis-0 scan of a row-major matrix).  Lines that ascend in memory in both
+// operands take the strips below (col_strip_kernel), very wide integer ones
+// and those that descend the single-pass col_lookback_kernel; this chunked
+// reduce-then-scan serves fewer than 256 descending lines, many short lines
+// (col_scan_kernel alone), and scans whose status words would not fit a
+// caller's fixed workspace (ScanArgs::small_workspace).  Lanes run across
+// lines -- a wave owns 64*V adjacent
 // lines, V = 4 giving every lane one 16-byte load per step -- and the scan
 // axis is cut into chunks so that thousands of waves share the work however
 // tall the matrix is:
@@ -1202,385 +1206,19 @@ __global__ __launch_bounds__(kBlock) void col_scan_kernel(ScanParams p, const ty
     }
 }
 
-// Narrow column scans: axis 0 of a dense row-major [R, C] matrix, C a power
-// of two from 32 to 128, read as the one contiguous range of 16-byte vectors
-// it is.  Component k of vector g holds column (4g + k) mod C, and since C
-// divides 256 that is column (4l + k) mod C for lane l of every step: a lane
-// always holds the same four columns, and the lanes of one column in a step
-// are l, l + s, l + 2s, ... with s = C / 4 (a "class").  A reverse scan
-// mirrors the range (logical vector g is physical vector nvec - 1 - g, its
-// components reversed), so every pass works in logical order and logical
-// columns.  Tiles are the scan's own: 8 waves x 16 steps of 64 vectors
-// (128 KiB, two blocks per CU), each wave streaming its own 16 KiB run with
-// all 16 loads in flight.  Three launches:
-//   col_narrow_totals_kernel  per tile and column, the total (one read);
-//   col_narrow_carry_kernel   per column, an exclusive scan of its totals;
-//   col_narrow_scan_kernel    every tile rescanned from its carries (one
-//                             read, one write).
-// f32 steps scan in f32 and add f64 carries; integers wrap.  The column-tile
-// forms gave such matrices one live lane in 64/C.  Narrower powers of two
-// take the single-pass row tiles (2^28 u32 at C = 4 / 8 / 16: 515 / 522 /
-// 525 us here, 439 / 450 / 455 there).
-constexpr int kNarrowWaves = 8, kNarrowSteps = 16;
-constexpr int kNarrowWavesPerEu = 4; // two 8-wave blocks per CU: at most 128 VGPRs
-constexpr uint64_t kNarrowTileVecs = (uint64_t)kNarrowWaves * kNarrowSteps * kWave;
-
-// Lane permutes for the class scans: lane l reads lane src(l), src given as
-// a byte address (4 * lane), 32-bit values.
-template <typename A> __device__ __forceinline__ A lane_permute(A v, int addr) {
-    static_assert(sizeof(A) == 4, "32-bit lanes");
-    return __builtin_bit_cast(A, __builtin_amdgcn_ds_bpermute(addr, __builtin_bit_cast(int, v)));
-}
-
-// Byte addresses of the lanes a class scan reads, per lane (S = C / 4 >= 2):
-// its class's last lane in the row below and in row 1 (S <= 16) or the lane
-// 32 below (S = 32), its class's last lane in the wave, and the lane S below.
-struct ClassLanes {
-    int below, row1, last, prev;
-    template <int S> __device__ __forceinline__ void init(int lane) {
-        const int c = lane & (S - 1);
-        if constexpr (S <= 16) {
-            below = 4 * (((lane & ~15) - S + c) & (kWave - 1));
-            row1 = 4 * (32 - S + c);
-        } else {
-            below = 4 * (lane & 31);
-            row1 = 0;
-        }
-        last = 4 * (kWave - S + c);
-        prev = 4 * ((lane - S) & (kWave - 1));
-    }
-};
-
-// Inclusive scan over the lanes of each class l mod S (S = 1, 2, 4, ..., 32):
-// lane l ends with the combination, in lane order, of the lanes l' <= l with
-// l' = l (mod S).  Distances S..8 inside each row of 16 lanes are DPP row
-// shifts; the class totals of lower rows then come in with two lane permutes
-// (rows 1 and 3 take their class's last lane of the row below; rows 2 and 3
-// then take its last lane of row 1).  S = 1 is the plain wave scan.  32-bit
-// values.
-template <int S, typename Op, typename A>
-__device__ __forceinline__ A class_inclusive_scan(A v, int lane, const ClassLanes &cl) {
-    if constexpr (S == 1) {
-        return wave_inclusive_scan<Op, A>(v);
-    } else {
-        const A id = Op::template identity<A>();
-        if constexpr (S <= 2) v = Op::combine(dpp_move<kDppRowShr2>(id, v), v);
-        if constexpr (S <= 4) v = Op::combine(dpp_move<kDppRowShr4>(id, v), v);
-        if constexpr (S <= 8) v = Op::combine(dpp_move<kDppRowShr8>(id, v), v);
-        if constexpr (S <= 16) {
-            const A below = lane_permute(v, cl.below);
-            v = (lane & 16) ? Op::combine(below, v) : v;
-            const A row1 = lane_permute(v, cl.row1);
-            v = lane >= 32 ? Op::combine(row1, v) : v;
-        } else {
-            const A half = lane_permute(v, cl.below);
-            v = lane >= 32 ? Op::combine(half, v) : v;
-        }
-        return v;
-    }
-}
-// The class total (the inclusive value of the class's last lane).
-template <int S, typename A> __device__ __forceinline__ A class_total(A incl, const ClassLanes &cl) {
-    if constexpr (S == 1) return read_lane(incl, kWave - 1);
-    else return lane_permute(incl, cl.last);
-}
-// Exclusive form: lane l takes lane l - S's inclusive value, the first S
-// lanes the identity.
-template <int S, typename Op, typename A>
-__device__ __forceinline__ A class_shift(A incl, int lane, const ClassLanes &cl) {
-    if constexpr (S == 1) {
-        return wave_shift_right<Op, A>(incl);
-    } else {
-        const A t = lane_permute(incl, cl.prev);
-        return lane >= S ? t : Op::template identity<A>();
-    }
-}
-
-// The rescan's in-wave part for class stride S, once the carries into the
-// wave are known (`outer`, per component): each step's components scanned
-// over their classes, and each output -- the carry, then the lane's running
-// class total before the step, then its (inclusive or exclusive) class
-// prefix -- handed to store(j, y) as soon as the step is scanned, so no
-// output is held in registers.  The running totals are in T: an f32 wave
-// prefix covers at most 16 steps of 64 values, and the carry is f64.
-template <int S, typename T, typename Op, bool EXCL, typename Store>
-__device__ __forceinline__ void narrow_wave_scan(const T (&x)[16][4], const typename ColAcc<T>::type (&outer)[4],
-                                                 int lane, Store &&store) {
-    using A = typename ColAcc<T>::type;
-    ClassLanes cl;
-    if constexpr (S > 1) cl.template init<S>(lane);
-    T run[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) run[k] = Op::template identity<T>();
-#pragma unroll
-    for (int j = 0; j < 16; ++j) {
-        T y[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const T incl = class_inclusive_scan<S, Op, T>(x[j][k], lane, cl);
-            const T tot = class_total<S, T>(incl, cl);
-            const T pre = EXCL ? class_shift<S, Op, T>(incl, lane, cl) : incl;
-            y[k] = (T)Op::combine(outer[k], (A)Op::combine(run[k], pre));
-            run[k] = Op::combine(run[k], tot);
-        }
-        store(j, y);
-    }
-}
-
-// Lane `lane`, wave `w` of tile `t`: its 16 logical vectors (steps j), whole
-// tiles through one block-uniform base and a 32-bit lane offset, the last
-// tile checked (identity past the end).
-template <typename T, bool REV>
-__device__ __forceinline__ void narrow_tile_load(const T *in, uint64_t nvec, uint64_t t, int w, int lane, T ident,
-                                                 T (&x)[kNarrowSteps][4]) {
-    using V = typename Vec4A4<T>::type;
-    const uint64_t g0 = t * kNarrowTileVecs + (uint64_t)w * (kNarrowSteps * kWave) + (uint64_t)lane;
-    if ((t + 1) * kNarrowTileVecs <= nvec) {
-        const uint32_t lane_off = ((uint32_t)__builtin_amdgcn_readfirstlane(w) * (kNarrowSteps * kWave) +
-                                   (uint32_t)lane) * 16u;
-        if constexpr (REV) {
-            const char *base = (const char *)(in + 4 * (nvec - (t + 1) * kNarrowTileVecs));
-            const uint32_t rev_off = (uint32_t)(kNarrowTileVecs * 16 - 16) - lane_off;
-#pragma unroll
-            for (int j = 0; j < kNarrowSteps; ++j) {
-                const V q = load_a4<true>((const V *)(base + rev_off - (uint32_t)j * (kWave * 16)));
-                x[j][0] = (T)q.w;
-                x[j][1] = (T)q.z;
-                x[j][2] = (T)q.y;
-                x[j][3] = (T)q.x;
-            }
-        } else {
-            const char *base = (const char *)(in + 4 * t * kNarrowTileVecs);
-#pragma unroll
-            for (int j = 0; j < kNarrowSteps; ++j) {
-                const V q = load_a4<true>((const V *)(base + lane_off + (uint32_t)j * (kWave * 16)));
-                x[j][0] = (T)q.x;
-                x[j][1] = (T)q.y;
-                x[j][2] = (T)q.z;
-                x[j][3] = (T)q.w;
-            }
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        return;
-    }
-#pragma unroll
-    for (int j = 0; j < kNarrowSteps; ++j) {
-        const uint64_t g = g0 + (uint64_t)j * kWave;
-        if (g < nvec) {
-            const V q = load_a4<true>((const V *)(in + 4 * (REV ? nvec - 1 - g : g)));
-            x[j][0] = (T)(REV ? q.w : q.x);
-            x[j][1] = (T)(REV ? q.z : q.y);
-            x[j][2] = (T)(REV ? q.y : q.z);
-            x[j][3] = (T)(REV ? q.x : q.w);
-        } else {
-#pragma unroll
-            for (int k = 0; k < 4; ++k) x[j][k] = ident;
-        }
-    }
-}
-
-// Pass 1: the totals of tile t, one per logical column, at totals[t * C + c].
-// Each lane folds its 16 steps per component, the lanes of a class fold with
-// xor butterflies from 32 down to s, and the waves' totals fold in wave
-// order: a fixed order, so f32 totals (accumulated in f64) are reproducible.
-template <typename T, typename Op, bool REV>
-__global__ __launch_bounds__(kNarrowWaves *kWave) void col_narrow_totals_kernel(ScanParams p,
-                                                                                typename ColAcc<T>::type *totals) {
-    using A = typename ColAcc<T>::type;
-    __shared__ A sh[kNarrowWaves][kBlock / 2]; // C <= 128 columns
-    const int lane = lane_id();
-    const int w = threadIdx.x / kWave;
-    const uint32_t C = (uint32_t)p.lines;
-    const uint32_t s = C / 4;
-    const uint64_t nvec = (p.len * C) >> 2;
-    const uint64_t t = xcd_contiguous(blockIdx.x, gridDim.x); // no look-back: any tile order
-    T x[kNarrowSteps][4];
-    narrow_tile_load<T, REV>((const T *)p.in + p.in_offset, nvec, t, w, lane, Op::template identity<T>(), x);
-    A acc[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        acc[k] = Op::template identity<A>();
-#pragma unroll
-        for (int j = 0; j < kNarrowSteps; ++j) acc[k] = Op::combine(acc[k], (A)x[j][k]);
-    }
-    for (int m = kWave / 2; m >= (int)s; m >>= 1)
-#pragma unroll
-        for (int k = 0; k < 4; ++k) acc[k] = Op::combine(acc[k], __shfl_xor(acc[k], m, kWave));
-    if (lane < (int)s)
-#pragma unroll
-        for (int k = 0; k < 4; ++k) sh[w][4 * lane + k] = acc[k];
-    __syncthreads();
-    for (uint32_t c = threadIdx.x; c < C; c += kNarrowWaves * kWave) {
-        A tot = Op::template identity<A>();
-#pragma unroll
-        for (int q = 0; q < kNarrowWaves; ++q) tot = Op::combine(tot, sh[q][c]);
-        totals[t * C + c] = tot;
-    }
-}
-
-// Pass 2: per column, the exclusive scan of the tile totals in place.  A
-// block per column; thread i owns a contiguous range of tiles, loaded 8 at a
-// time with the loads of a batch in flight together (one batch, held in
-// registers, for up to 8192 tiles), its range total scanned across the block
-// in thread order, and its range rewritten.  The order depends only on the
-// tile count, so f32 carries are reproducible.  (Re-reading each value in the
-// rewrite loop made every iteration a dependent memory round trip: 17-25 us
-// per launch.)
-constexpr int kNarrowCarryThreads = 1024;
-constexpr int kNarrowCarryBatch = 8;
-// Entry (tile k, column c) is totals[k * ks + c * cs]: row-major (ks = C,
-// cs = 1) for the narrow form, column-major (ks = 1, cs = tiles) for the row
-// tiles, whose carry launch read row-major totals C words apart (2^28 u32 at
-// C = 100 and 255, about 16400 tiles: 76 us per launch).
-template <typename A, typename Op>
-__global__ __launch_bounds__(kNarrowCarryThreads) void col_narrow_carry_kernel(A *totals, uint64_t ks, uint64_t cs,
-                                                                               uint64_t ntiles) {
-    __shared__ A sh[kNarrowCarryThreads / kWave];
-    A *col = totals + (uint64_t)blockIdx.x * cs;
-    const int lane = lane_id();
-    const int w = threadIdx.x / kWave;
-    const uint64_t per = (ntiles + kNarrowCarryThreads - 1) / kNarrowCarryThreads;
-    const uint64_t k0 = (uint64_t)threadIdx.x * per < ntiles ? (uint64_t)threadIdx.x * per : ntiles;
-    const uint64_t k1 = k0 + per < ntiles ? k0 + per : ntiles;
-    const A id = Op::template identity<A>();
-    A v[kNarrowCarryBatch];
-    A sum = id;
-    for (uint64_t k = k0; k < k1; k += kNarrowCarryBatch) {
-#pragma unroll
-        for (int u = 0; u < kNarrowCarryBatch; ++u) v[u] = k + u < k1 ? col[(k + u) * ks] : id;
-#pragma unroll
-        for (int u = 0; u < kNarrowCarryBatch; ++u) sum = Op::combine(sum, v[u]);
-    }
-    // Exclusive scan of the range totals in thread order: within each wave,
-    // then the wave totals through LDS.
-    A incl = sum;
-#pragma unroll
-    for (int d = 1; d < kWave; d <<= 1) {
-        const A t = __shfl_up(incl, d, kWave);
-        if (lane >= d) incl = Op::combine(t, incl);
-    }
-    if (lane == kWave - 1) sh[w] = incl;
-    __syncthreads();
-    A acc = id;
-    for (int q = 0; q < w; ++q) acc = Op::combine(acc, sh[q]);
-    const A prev = __shfl_up(incl, 1, kWave);
-    if (lane > 0) acc = Op::combine(acc, prev);
-    for (uint64_t k = k0; k < k1; k += kNarrowCarryBatch) {
-        if (per > kNarrowCarryBatch) { // the range spans several batches: reload this one
-#pragma unroll
-            for (int u = 0; u < kNarrowCarryBatch; ++u) v[u] = k + u < k1 ? col[(k + u) * ks] : id;
-        }
-#pragma unroll
-        for (int u = 0; u < kNarrowCarryBatch; ++u) {
-            if (k + u < k1) col[(k + u) * ks] = acc;
-            acc = Op::combine(acc, v[u]);
-        }
-    }
-}
-
-// Pass 3: tile t rescanned from its columns' carries (pass 2), or from the
-// identity for a single tile.  Each wave first folds its column totals (per
-// lane over its 16 steps, then across the lanes of a class), the waves'
-// totals combine with the tile's carries through LDS in wave order, and only
-// then are the steps scanned (narrow_wave_scan), every step stored as soon as
-// it is scanned: holding the outputs until the carries were known took
-// 140-145 VGPRs, one block per CU.  Whole tiles store through the
-// stream-store path, the last tile element by element.
-template <typename T, typename Op, bool EXCL, bool REV, bool CARRY>
-__global__ __launch_bounds__(kNarrowWaves *kWave) __attribute__((amdgpu_waves_per_eu(kNarrowWavesPerEu)))
-void col_narrow_scan_kernel(ScanParams p, const typename ColAcc<T>::type *carries) {
-    using A = typename ColAcc<T>::type;
-    using V = typename Vec4A4<T>::type;
-    __shared__ A sh[kNarrowWaves][kBlock / 2]; // C <= 128 columns
-    const int lane = lane_id();
-    const int w = threadIdx.x / kWave;
-    const uint32_t C = (uint32_t)p.lines;
-    const uint32_t s = C / 4;
-    const uint64_t nvec = (p.len * C) >> 2;
-    const uint64_t t = xcd_contiguous(blockIdx.x, gridDim.x); // no look-back: any tile order
-    T x[kNarrowSteps][4];
-    narrow_tile_load<T, REV>((const T *)p.in + p.in_offset, nvec, t, w, lane, Op::template identity<T>(), x);
-
-    // The wave's column totals, then per column the carry into each wave.
-    A acc[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        acc[k] = Op::template identity<A>();
-#pragma unroll
-        for (int j = 0; j < kNarrowSteps; ++j) acc[k] = Op::combine(acc[k], (A)x[j][k]);
-    }
-    for (int m = kWave / 2; m >= (int)s; m >>= 1)
-#pragma unroll
-        for (int k = 0; k < 4; ++k) acc[k] = Op::combine(acc[k], __shfl_xor(acc[k], m, kWave));
-    if (lane < (int)s)
-#pragma unroll
-        for (int k = 0; k < 4; ++k) sh[w][4 * lane + k] = acc[k];
-    __syncthreads();
-    if (threadIdx.x < C) {
-        A c = CARRY ? carries[t * C + threadIdx.x] : Op::template identity<A>();
-#pragma unroll
-        for (int q = 0; q < kNarrowWaves; ++q) {
-            const A v = sh[q][threadIdx.x];
-            sh[q][threadIdx.x] = c;
-            c = Op::combine(c, v);
-        }
-    }
-    __syncthreads();
-    A outer[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) outer[k] = sh[w][(uint32_t)(4 * lane + k) & (C - 1)];
-
-    T *out = (T *)p.out + p.out_offset;
-    const bool full = (t + 1) * kNarrowTileVecs <= nvec;
-    const uint32_t lane_off =
-        ((uint32_t)__builtin_amdgcn_readfirstlane(w) * (kNarrowSteps * kWave) + (uint32_t)lane) * 16u;
-    const uint32_t rev_off = (uint32_t)(kNarrowTileVecs * 16 - 16) - lane_off;
-    const auto orsrc = stream_rsrc(out + 4 * (REV ? (full ? nvec - (t + 1) * kNarrowTileVecs : 0)
-                                                   : t * kNarrowTileVecs),
-                                   (uint32_t)(kNarrowTileVecs * 16));
-    const uint64_t g0 = t * kNarrowTileVecs + (uint64_t)w * (kNarrowSteps * kWave) + (uint64_t)lane;
-    auto store = [&](int j, const T (&y)[4]) {
-        V v;
-        v.x = REV ? y[3] : y[0];
-        v.y = REV ? y[2] : y[1];
-        v.z = REV ? y[1] : y[2];
-        v.w = REV ? y[0] : y[3];
-        if (full) {
-            stream_store(v, orsrc, REV ? rev_off - (uint32_t)j * (kWave * 16) : lane_off + (uint32_t)j * (kWave * 16));
-        } else {
-            const uint64_t g = g0 + (uint64_t)j * kWave;
-            if (g < nvec) store_a4<true>(v, (V *)(out + 4 * (REV ? nvec - 1 - g : g)));
-        }
-    };
-    switch (s) { // wave-uniform: C is a launch parameter
-    case 8: narrow_wave_scan<8, T, Op, EXCL>(x, outer, lane, store); break;
-    case 16: narrow_wave_scan<16, T, Op, EXCL>(x, outer, lane, store); break;
-    default: narrow_wave_scan<32, T, Op, EXCL>(x, outer, lane, store); break;
-    }
-}
-
-// Row-tile column scans: axis 0 of a dense row-major [R, C] matrix for the
-// other column counts from 2 to 255 (every C but 32, 64 and 128).  Unless C
-// divides 256 the 16-byte lanes of the narrow form would not see fixed
-// columns.  Up to kRowTileLbMaxCols columns the tiles look back in one pass
-// (col_rowtile_lookback_kernel, below); wider matrices take three.  A tile
-// of `rows` whole rows (a multiple of 4, at most kRowTileElems elements)
-// moves between HBM and LDS as coalesced 16-byte vectors.  In LDS, thread j
-// owns column j mod C over row group j / C, one of G = 512 / C contiguous
-// groups of `rpg` rows: pass 1 (col_rowtile_totals_kernel) folds each group,
-// then scans the group totals along the groups (row_group_scan), whose last
-// group holds the tile's column totals; pass 2 is
-// col_narrow_carry_kernel; pass 3 (col_rowtile_scan_kernel) folds the
-// groups again, then rescans each group's rows in place from the tile's
-// carry and the earlier groups' totals before the tile is stored.  Every
-// combination runs in ColAcc (f64 for f32) in an order fixed by the shape,
-// so f32 results are reproducible.  Mirrored scans take tiles from row R - 1
+// Row-tile column scans: axis 0 of a dense row-major [R, C] matrix of 2 to 24
+// columns, where a strip's lanes would mostly be idle.  A tile of `rows`
+// whole rows (a multiple of 4, at most kRowTileElems elements) moves between
+// HBM and LDS as coalesced 16-byte vectors.  In LDS, thread j owns column j
+// mod C over row group j / C, one of G = 512 / C contiguous groups of `rpg`
+// rows: it folds its group, the group totals are scanned along the groups
+// (row_group_scan), whose last group holds the tile's column totals, and
+// after the look-back it rescans its rows in place from the tile's carry and
+// the earlier groups' totals before the tile is stored.  Every combination
+// runs in ColAcc (f64 for f32).  Mirrored scans take tiles from row R - 1
 // down and walk each tile's rows upwards in LDS.  The strided per-line path
 // gave these shapes one lane per line (2^28 u32, C = 3: 2.3 ms; C = 12:
-// 10 ms).  Tiles of 16384 elements and 512 threads (two blocks per CU by
-// LDS) measured best: 2^28 u32 at C = 3 / 12 / 100 / 255 took 597 / 586 /
-// 592 / 638 us, against 614 / 594 / 656 / 712 with 8192 elements and 256
-// threads and 651 / 682 / 820 / 906 with 4096.
+// 10 ms).
 constexpr int kRowTileThreads = 512;
 constexpr uint32_t kRowTileElems = 16384;
 constexpr int kRowTileVecsPerThread = (int)(kRowTileElems / 4 / kRowTileThreads);
@@ -1708,60 +1346,6 @@ __device__ __forceinline__ void row_group_rescan(T *tile, uint32_t n, uint32_t C
     }
 }
 
-template <typename T, typename Op, bool REV>
-__global__ __launch_bounds__(kRowTileThreads) __attribute__((amdgpu_waves_per_eu(4))) void col_rowtile_totals_kernel(ScanParams p, RowTileShape s,
-                                                                             typename ColAcc<T>::type *totals) {
-    using A = typename ColAcc<T>::type;
-    __shared__ __attribute__((aligned(16))) T tile[kRowTileElems];
-    __shared__ A gtot[kRowTileThreads];
-    const uint64_t t = xcd_contiguous(blockIdx.x, gridDim.x); // no look-back: any tile order
-    const uint32_t C = s.C;
-    uint64_t r0;
-    uint32_t n;
-    row_tile_span<REV>(s, t, r0, n);
-    row_tile_load<T>((const T *)p.in + p.in_offset + r0 * C, n * C, tile);
-    __syncthreads();
-    const uint32_t j = threadIdx.x, g = j / C, c = j - g * C;
-    const bool owner = g < s.groups;
-    if (owner) {
-        const uint32_t lo = g * s.rpg < n ? g * s.rpg : n;
-        const uint32_t hi = lo + s.rpg < n ? lo + s.rpg : n;
-        gtot[j] = row_group_fold<T, Op, REV>(tile, n, C, c, lo, hi);
-    }
-    __syncthreads();
-    row_group_scan<A, Op>(gtot, s.groups, C, j, owner, g);
-    if (j < C) totals[(uint64_t)j * s.tiles + t] = gtot[(s.groups - 1) * C + j]; // column-major
-}
-
-template <typename T, typename Op, bool EXCL, bool REV, bool CARRY>
-__global__ __launch_bounds__(kRowTileThreads) __attribute__((amdgpu_waves_per_eu(4))) void col_rowtile_scan_kernel(ScanParams p, RowTileShape s,
-                                                                           const typename ColAcc<T>::type *carries) {
-    using A = typename ColAcc<T>::type;
-    __shared__ __attribute__((aligned(16))) T tile[kRowTileElems];
-    __shared__ A gtot[kRowTileThreads];
-    const uint64_t t = xcd_contiguous(blockIdx.x, gridDim.x); // no look-back: any tile order
-    const uint32_t C = s.C;
-    uint64_t r0;
-    uint32_t n;
-    row_tile_span<REV>(s, t, r0, n);
-    row_tile_load<T>((const T *)p.in + p.in_offset + r0 * C, n * C, tile);
-    __syncthreads();
-    const uint32_t j = threadIdx.x, g = j / C, c = j - g * C;
-    const bool owner = g < s.groups;
-    const uint32_t lo = g * s.rpg < n ? g * s.rpg : n;
-    const uint32_t hi = lo + s.rpg < n ? lo + s.rpg : n;
-    if (owner) gtot[j] = row_group_fold<T, Op, REV>(tile, n, C, c, lo, hi);
-    __syncthreads();
-    row_group_scan<A, Op>(gtot, s.groups, C, j, owner, g);
-    if (owner) {
-        A pre = CARRY ? carries[(uint64_t)c * s.tiles + t] : Op::template identity<A>();
-        if (g > 0) pre = Op::combine(pre, gtot[j - C]);
-        row_group_rescan<T, Op, EXCL, REV>(tile, n, C, c, lo, hi, pre);
-    }
-    __syncthreads();
-    row_tile_store<T>(tile, n * C, (T *)p.out + p.out_offset + r0 * C);
-}
-
 // Single-pass row-tile column scan: the row tiles above with a decoupled
 // look-back over C-wide carries, so every element is read once and written
 // once.  Status entry (tile u, column c) is u * C + c.  After its groups'
@@ -1776,14 +1360,13 @@ __global__ __launch_bounds__(kRowTileThreads) __attribute__((amdgpu_waves_per_eu
 // to rounding) and uses it, so progress never depends on dispatch order.  The round's needed values fold over k through an LDS tree
 // into the column carry, which is published with the tile's aggregate as the
 // inclusive prefix.  Tile 0's value is always its prefix.  f32 carries are
-// f64 in 16-byte slots (F64QuadDense), integers packed words.  Unlike the
-// three-pass form, an f32 carry's f64 rounding depends on which predecessors
-// had published prefixes: results agree with the f64 scan to within its
-// bound, not bit for bit across runs.  2^28 u32, us, three passes -> one:
-// C = 2 556 -> 474, 3 599 -> 471, 7 608 -> 473, 12 606 -> 468, 24 579 ->
-// 514; at C = 48 / 100 / 255 (a round covering 10 / 5 / 2 predecessors)
-// one pass took 622 / 800 / 1093, and several statuses per thread and
-// round (up to 8) 572 / 687 / 909 against 578 / 585 / 635 in three passes.
+// f64 in 16-byte slots (F64QuadDense), integers packed words.  An f32
+// carry's f64 rounding depends on which predecessors had published prefixes:
+// results agree with the f64 scan to within its bound, not bit for bit across
+// runs.  2^28 u32, us, against totals, carries and a rescan in three
+// launches: C = 2 556 -> 474, 3 599 -> 471, 7 608 -> 473, 12 606 -> 468, 24
+// 579 -> 514; at C = 48 / 100 / 255 (a round covering 10 / 5 / 2
+// predecessors) one pass of these tiles took 622 / 800 / 1093.
 template <typename T, typename Op, bool REV>
 __device__ __forceinline__ typename ColAcc<T>::type rowtile_column_aggregate(const ScanParams &p, const RowTileShape &s,
                                                                          uint64_t u, uint32_t c) {
@@ -2227,6 +1810,281 @@ __global__ __launch_bounds__(kColWaves *kWave) void col_lookback_kernel(ScanPara
     }
 }
 
+// Strip column scans: many lines adjacent in memory (axis 0 of a row-major
+// matrix), read and written once.  The lines are cut into strips of W (32 or
+// 64) and the scan axis into chunks; a block owns one chunk of one strip.  Its
+// data waves put W / 4 lanes on a row (one 16-byte vector of four lines each)
+// and 256 / W rows on a load instruction; a lane takes STEPS consecutive rows
+// and keeps them in registers.  The lanes' totals go to LDS, and the block's
+// last wave, which holds no data, turns them into the lanes' exclusive
+// prefixes (a lane per line), publishes the chunk's totals and looks back over
+// the strip's earlier chunks, P statuses per line in flight, while the data
+// waves wait at the barrier; each lane then rescans its rows from the carry.
+// Integers wrap in u32; f32 totals, carries and running values are all f64.
+//
+// Why strips: a look-back's length is the number of chunks that load at the
+// same time, and its cost one round trip (1.5 to 2.5 us) per P chunks.  A
+// strip of 64 lines leaves room for 448 rows in a block of 8 waves, against
+// 240 rows of 256 lines in the 16-wave tiles of col_lookback_kernel, and gives
+// a matrix four times as many chains.  Below 256 lines it replaces three
+// passes (totals, carries, rescan), 12 bytes an element instead of 8.
+// Measured on MI355X, 2^26 elements, u32 / f32, us: [2^21, 32] 139 / 141 ->
+// 85 / 111; [2^20, 64] 139 / 143 -> 85 / 105; [2^19, 128] 142 / 145 -> 89 / 99;
+// [65536, 1024] 102 / 130 -> 100 / 99; smaller, u32: [510, 659] 11.8 -> 5.4,
+// [1146, 90] 12.0 -> 5.4, [4096, 1024] 16.9 -> 8.3.
+//
+// Whole 128-byte lines (row pitch and output start multiples of 128 bytes)
+// are stored non-temporally.  Elsewhere neighbouring strips share the lines
+// at their edges, and a non-temporal store of part of a line costs a
+// read-modify-write in memory: such strips store through the L2, and the
+// blocks are dealt so that the strips that share lines run on one XCD, whose
+// L2 then merges the parts (StripDeal).  [700001, 100] u32: 193 us
+// non-temporal, 139 through the L2, 110 with the deal (three passes: 148);
+// [165595, 486] f32 229, 185, 135 (183).
+enum StripDeal : uint32_t {
+    kDealRows = 0,   // block b: strip b mod groups of chunk b / groups
+    kDealChunks = 1, // every chunk's strips on one XCD, chunks round robin
+    kDealStrips = 2, // an eighth of the strips on each XCD
+};
+
+constexpr int kStripWaves = 8;
+template <int W, int STEPS> struct StripGeom {
+    static_assert(W == 32 || W == 64, "strips of 32 or 64 lines");
+    static constexpr int kDataWaves = kStripWaves - 1;
+    static constexpr int kLanesPerRow = W / 4;
+    static constexpr int kSub = kWave / kLanesPerRow; // rows per load instruction
+    static constexpr int kParts = kDataWaves * kSub;  // lanes along the axis
+    static constexpr uint64_t kRows = (uint64_t)kParts * STEPS;
+};
+
+// Statuses in flight per line: the f32 slots are 16 bytes, and four of them
+// a line took [2^19, 128] from 99 us to 103.
+template <typename T> struct StripPolls { static constexpr int value = 4; };
+template <> struct StripPolls<float> { static constexpr int value = 2; };
+
+// The last wave's look-back: lane l < W (live where the line exists) folds
+// its line's statuses of the chunks before `c`, nearest first, P per round
+// trip, consumed in order and in step for the whole wave, and publishes the
+// line's inclusive prefix.  Entry (chunk, line) of the status array is
+// chunk * lpad + entry.  A chunk that stays unpublished for p.spin_limit polls
+// is totalled from the input by the waiter, so progress never depends on the
+// dispatch order; the value is not published (every slot has one writer).
+template <typename T, typename Op, typename Status, uint64_t ROWS, bool REV>
+__device__ void strip_lookback(const ScanParams &p, const Status &st, uint64_t c, uint64_t lpad, uint64_t line,
+                               uint64_t entry, bool live, typename ColAcc<T>::type agg,
+                               typename ColAcc<T>::type &excl) {
+    using A = typename ColAcc<T>::type;
+    constexpr int P = StripPolls<T>::value;
+    excl = Op::template identity<A>();
+    if (c == 0) {
+        if (live) st.publish_tile(entry, p.tag, kPrefix, agg);
+        return;
+    }
+    if (live) st.publish_tile(c * lpad + entry, p.tag, kAggregate, agg);
+    bool done = !live;
+    uint64_t pos = c - 1; // next chunk to consume
+    uint32_t spins = 0;
+    for (;;) {
+        uint32_t flag[P];
+        A val[P];
+        // Every lane reads (chunk 0 past the start): straight-line loads stay
+        // in flight together.
+#pragma unroll
+        for (int k = 0; k < P; ++k)
+            st.read((pos >= (uint64_t)k ? pos - k : 0) * lpad + entry, p.tag, flag[k], val[k]);
+        uint32_t used = 0;
+        bool finished = false;
+#pragma unroll
+        for (int k = 0; k < P; ++k) {
+            if (finished || used != (uint32_t)k || pos < (uint64_t)k) continue;
+            if (ballot(!done && flag[k] == kInvalid) != 0ull) continue;
+            if (!done) {
+                excl = Op::combine(val[k], excl);
+                done = flag[k] == kPrefix || pos == (uint64_t)k; // chunk 0 ends every line
+            }
+            used = k + 1;
+            finished = ballot(!done) == 0ull;
+        }
+        if (finished) break;
+        pos -= used; // chunk 0 finishes, so used <= pos here
+        if (used != 0) {
+            spins = 0;
+            continue;
+        }
+        if (++spins < p.spin_limit) {
+            __builtin_amdgcn_s_sleep(1);
+            continue;
+        }
+        spins = 0;
+        A t = Op::template identity<A>();
+        if (live) {
+            const T *in = (const T *)p.in + ((int64_t)p.in_offset + (int64_t)line);
+#pragma unroll 8
+            for (uint64_t i = pos * ROWS; i < (pos + 1) * ROWS; ++i) // earlier chunks are whole
+                t = Op::combine(t, (A)in[(int64_t)(REV ? p.len - 1 - i : i) * p.in_elem_stride]);
+        }
+        if (!done) {
+            const bool missing = flag[0] == kInvalid;
+            excl = Op::combine(missing ? t : val[0], excl);
+            done = (!missing && flag[0] == kPrefix) || pos == 0;
+        }
+        if (ballot(!done) == 0ull) break;
+        pos -= 1;
+    }
+    if (live) st.publish_tile(c * lpad + entry, p.tag, kPrefix, Op::combine(excl, agg));
+}
+
+struct StripParams {
+    uint32_t groups, width; // strips, lines per strip (a multiple of 4, at most W)
+    uint32_t deal;          // StripDeal
+    uint32_t cached;        // stores go through the L2 (else non-temporal)
+    uint64_t lpad;          // status entries per chunk
+    uint64_t chunks;
+};
+
+template <typename T, typename Op, typename Status, int W, int STEPS, bool EXCL, bool REV>
+__global__ __launch_bounds__(kStripWaves *kWave) __attribute__((amdgpu_waves_per_eu(4)))
+void col_strip_kernel(ScanParams p, StripParams sp, Status st) {
+    using A = typename ColAcc<T>::type;
+    using G = StripGeom<W, STEPS>;
+    using Vt = typename Vec4A4<T>::type;
+    __shared__ A s_part[G::kParts][W]; // lane totals, then their exclusive prefixes
+    __shared__ A s_carry[W];
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int lane = lane_id();
+    // Predecessor chunks always have lower block indices.
+    uint32_t g;
+    uint64_t c;
+    if (sp.deal == kDealRows) {
+        g = blockIdx.x % sp.groups;
+        c = blockIdx.x / sp.groups;
+    } else {
+        const uint32_t xcd = blockIdx.x % kXcds, q = blockIdx.x / kXcds;
+        if (sp.deal == kDealChunks) {
+            g = q % sp.groups;
+            c = (uint64_t)(q / sp.groups) * kXcds + xcd;
+        } else {
+            const uint32_t per = (sp.groups + kXcds - 1) / kXcds;
+            g = xcd * per + q % per;
+            c = q / per;
+        }
+        if (g >= sp.groups || c >= sp.chunks) return; // the deal's padding
+    }
+    const uint64_t first = (uint64_t)g * sp.width; // the strip's first line
+    const uint32_t cnt = p.lines - first < sp.width ? (uint32_t)(p.lines - first) : sp.width;
+    const A aid = Op::template identity<A>();
+
+    if (w == G::kDataWaves) {
+        __syncthreads(); // the lanes' totals
+        const int l = lane & (W - 1);
+        A run = aid;
+        if (lane < W) {
+#pragma unroll 14
+            for (int e = 0; e < G::kParts; ++e) {
+                const A v = s_part[e][l];
+                s_part[e][l] = run;
+                run = Op::combine(run, v);
+            }
+        }
+        A excl;
+        strip_lookback<T, Op, Status, G::kRows, REV>(p, st, c, sp.lpad, first + l, (uint64_t)g * W + l,
+                                                     lane < (int)cnt, run, excl);
+        if (lane < W) s_carry[l] = excl;
+        __syncthreads(); // the carry
+        return;
+    }
+
+    const uint32_t sub = (uint32_t)lane / G::kLanesPerRow, q = (uint32_t)lane % G::kLanesPerRow;
+    // Lane q's lines l0 .. l0 + nv - 1 of the strip.  Where the strip's line
+    // count is no multiple of 4 its last lane moves back to a whole vector: the
+    // lines it shares with its neighbour get the same values twice.
+    const bool active = 4 * q < cnt;
+    const uint32_t l0 = cnt < 4 ? 0u : 4 * q + 4 <= cnt ? 4 * q : cnt - 4;
+    const uint32_t nv = active ? (cnt < 4 ? cnt : 4u) : 0u;
+    const uint32_t part = (uint32_t)w * G::kSub + sub;
+    const uint64_t i0 = c * G::kRows + (uint64_t)part * STEPS;
+    const bool whole = (c + 1) * G::kRows <= p.len;
+    const T tid = Op::template identity<T>();
+    T x[STEPS][4];
+    {
+        const T *src = (const T *)p.in + ((int64_t)p.in_offset + (int64_t)(first + l0) +
+                                          (int64_t)(REV ? p.len - 1 - i0 : i0) * p.in_elem_stride);
+        const int64_t step = REV ? -p.in_elem_stride : p.in_elem_stride;
+        if (whole && nv == 4) {
+#pragma unroll
+            for (int j = 0; j < STEPS; ++j) {
+                col_load_t<T, 4>(src, x[j]);
+                src += step;
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < STEPS; ++j) {
+                if (active && i0 + j < p.len) {
+                    col_load_n<T, 4>(src, nv, tid, x[j]);
+                } else {
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) x[j][v] = tid;
+                }
+                src += step;
+            }
+        }
+    }
+    {
+        A tot[4];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) tot[v] = aid;
+#pragma unroll
+        for (int j = 0; j < STEPS; ++j)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) tot[v] = Op::combine(tot[v], (A)x[j][v]);
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+            if ((uint32_t)v < nv) s_part[part][l0 + v] = tot[v];
+    }
+    __syncthreads(); // totals to the last wave
+    __syncthreads(); // its prefixes and carry
+    if (!active) return;
+    A run[4];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        const uint32_t l = (uint32_t)v < nv ? l0 + v : l0;
+        run[v] = Op::combine(s_carry[l], s_part[part][l]);
+    }
+    T *dst = (T *)p.out + ((int64_t)p.out_offset + (int64_t)(first + l0) +
+                           (int64_t)(REV ? p.len - 1 - i0 : i0) * p.out_elem_stride);
+    const int64_t step = REV ? -p.out_elem_stride : p.out_elem_stride;
+#pragma unroll
+    for (int j = 0; j < STEPS; ++j) {
+        if (!whole && i0 + j >= p.len) break;
+        T y[4];
+        // Opaque: the totals' f64 conversions are not kept for this second
+        // use (they would hold 128 registers across the look-back).
+#pragma unroll
+        for (int v = 0; v < 4; ++v) asm volatile("" : "+v"(x[j][v]));
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            if constexpr (EXCL) y[v] = (T)run[v];
+            run[v] = Op::combine(run[v], (A)x[j][v]);
+            if constexpr (!EXCL) y[v] = (T)run[v];
+        }
+        if (!sp.cached) {
+            col_store_n<T, 4>(dst, nv, y);
+        } else if (nv == 4) {
+            Vt v;
+            v.x = y[0];
+            v.y = y[1];
+            v.z = y[2];
+            v.w = y[3];
+            *(Vt *)dst = v;
+        } else {
+#pragma unroll
+            for (int v = 0; v < 3; ++v)
+                if ((uint32_t)v < nv) dst[v] = y[v];
+        }
+        dst += step;
+    }
+}
+
 // 16 waves per CU: on a 65536 x 4096 u32 column scan 4096 waves of 256 steps
 // took 164 + 12 + 386 us (totals, carry, rescan); 8192 waves 202 + 23 + 512.
 constexpr uint64_t kColTargetWaves = 4096;
@@ -2284,11 +2142,10 @@ ColLbShape col_lb_shape(const ScanArgs &a) {
     return s;
 }
 
-// The single pass needs whole line groups: with fewer than 256 lines every
-// tile leaves lanes idle and all tiles form one long look-back chain
+// col_lookback_kernel needs whole line groups: with fewer than 256 lines
+// every tile leaves lanes idle and all tiles form one long look-back chain
 // (measured, u32: 4194304 x 64 1.63 ms single-pass against 0.75 ms chunked;
-// 1048576 x 256 0.46 against 0.71; 65536 x 4096 0.35 against 0.54; f32
-// 65536 x 4096 0.48 against 0.56).
+// 1048576 x 256 0.46 against 0.71; 65536 x 4096 0.35 against 0.54).
 constexpr uint64_t kSinglePassMinLines = 256;
 // Many short lines: a scan of at most kColShortMaxLen steps whose chunked
 // form needs one chunk over at least kColShortMinGroups line groups reads and
@@ -2301,10 +2158,30 @@ constexpr uint64_t kSinglePassMinLines = 256;
 // serial steps ([32, 2^16]: 5.3 us against 7.5).
 constexpr uint64_t kColShortMaxLen = 64;
 constexpr uint64_t kColShortMinGroups = 1024;
-bool column_single_pass(const ScanArgs &a) {
+bool column_short_lines(const ScanArgs &a) {
     if (!column_mode(a) || a.lines < kSinglePassMinLines) return false;
     const ColShape s = column_shape(a);
-    return !(s.nchunks == 1 && a.len <= kColShortMaxLen && s.groups >= kColShortMinGroups);
+    return s.nchunks == 1 && a.len <= kColShortMaxLen && s.groups >= kColShortMinGroups;
+}
+// Large integer matrices keep col_lookback_kernel's 1 KiB rows against the
+// strips' 256 bytes, from 1024 lines where the rows are whole 128-byte lines
+// and from 4096 where they are whole 16-byte vectors: u32, us, [32768, 4096]
+// 182 against 195, [131072, 1024] 189 against 201, [49152, 2048] 146 against
+// 153, [26541, 4532] 205 against 211; but [524288, 256] 250 against 200, [65536,
+// 1024] 102 against 91, [30000, 5001] 275 against 267.
+constexpr uint64_t kWideLines = 1024, kWideVectorLines = 4096;
+constexpr uint64_t kWideElems = 1ull << 26;
+bool whole_line_rows(const ScanArgs &a) {
+    return ((uintptr_t)a.out + 4u * a.out_offset) % 128 == 0 && a.out_elem_stride % 32 == 0; // 4-byte elements
+}
+bool column_wide(const ScanArgs &a) {
+    if (a.dtype == HX_DTYPE_F32 || a.len * a.lines <= kWideElems) return false;
+    return (a.lines >= kWideLines && whole_line_rows(a)) ||
+           (a.lines >= kWideVectorLines && a.out_elem_stride % 4 == 0);
+}
+bool column_single_pass(const ScanArgs &a) {
+    return column_mode(a) && a.lines >= kSinglePassMinLines && !a.small_workspace && !column_short_lines(a) &&
+           (column_shape(a).V == 1 || column_wide(a));
 }
 
 uint64_t column_bytes(const ScanArgs &a) {
@@ -2357,9 +2234,9 @@ template <typename T, typename Op>
 hx_status launch_col_lookback(const ScanParams &p, const ColLbShape &s, bool excl, bool rev, void *status,
                               hipStream_t stream) {
     if constexpr (std::is_same<T, float>::value) {
+        // Ascending f32 lines take the strips (column_single_pass).
         const F64PairStatus st{(uint64_t *)status};
-        return s.V == 4 ? launch_col_lookback_s<T, Op, F64PairStatus, 4>(p, s, st, excl, rev, stream)
-                        : launch_col_lookback_s<T, Op, F64PairStatus, 1>(p, s, st, excl, rev, stream);
+        return launch_col_lookback_s<T, Op, F64PairStatus, 1>(p, s, st, excl, rev, stream);
     } else {
         const PackedStatus st{(uint64_t *)status};
         return s.V == 4 ? launch_col_lookback_s<T, Op, PackedStatus, 4>(p, s, st, excl, rev, stream)
@@ -2512,100 +2389,16 @@ hx_status launch_short(const ScanArgs &a, hipStream_t stream) {
     return a.reverse ? launch_short_dir<T, Op, false, true>(p, stream) : launch_short_dir<T, Op, false, false>(p, stream);
 }
 
-// Narrow column scans (col_narrow_*): see the kernels' comment.
-bool narrow_column_scan(const ScanArgs &a) {
-    const uint64_t c = a.lines;
-    const uintptr_t ibase = (uintptr_t)a.in + 4u * a.in_offset; // every element type is 4 bytes
-    const uintptr_t obase = (uintptr_t)a.out + 4u * a.out_offset;
-    return c >= 32 && c < kSinglePassMinLines && (c & (c - 1)) == 0 && a.in_line_stride == 1 &&
-           a.out_line_stride == 1 && a.in_elem_stride == (int64_t)c && a.out_elem_stride == (int64_t)c &&
-           ibase % 4 == 0 && obase % 4 == 0;
-}
-
-uint64_t narrow_tiles(const ScanArgs &a) { return ceil_div((a.len * a.lines) >> 2, kNarrowTileVecs); }
-uint64_t narrow_bytes(const ScanArgs &a) {
-    const uint64_t tiles = narrow_tiles(a);
-    if (tiles <= 1) return 0;
-    return tiles * a.lines * (a.dtype == HX_DTYPE_F32 ? 8u : 4u);
-}
-
-template <typename T, typename Op, bool EXCL, bool REV>
-hx_status launch_narrow_dir(const ScanParams &p, uint64_t tiles, void *ws, hipStream_t stream) {
-    using A = typename ColAcc<T>::type;
-    if (tiles > 0x7FFFFFFFull) return fail(HX_ERR_DISPATCH_FAILED, "column scan exceeds the grid range");
-    const dim3 grid((uint32_t)tiles), block(kNarrowWaves * kWave);
-    A *totals = (A *)ws;
-    if (tiles > 1) {
-        hipLaunchKernelGGL((col_narrow_totals_kernel<T, Op, REV>), grid, block, 0, stream, p, totals);
-        HX_TRY(check_launch("col_narrow_totals_kernel"));
-        hipLaunchKernelGGL((col_narrow_carry_kernel<A, Op>), dim3((uint32_t)p.lines), dim3(kNarrowCarryThreads), 0,
-                           stream, totals, p.lines, (uint64_t)1, tiles);
-        HX_TRY(check_launch("col_narrow_carry_kernel"));
-        hipLaunchKernelGGL((col_narrow_scan_kernel<T, Op, EXCL, REV, true>), grid, block, 0, stream, p,
-                           (const A *)totals);
-    } else {
-        hipLaunchKernelGGL((col_narrow_scan_kernel<T, Op, EXCL, REV, false>), grid, block, 0, stream, p,
-                           (const A *)totals);
-    }
-    return check_launch("col_narrow_scan_kernel");
-}
-
-template <typename T, typename Op>
-hx_status launch_narrow(const ScanArgs &a, const ScanParams &p, void *ws, uint64_t ws_bytes, hipStream_t stream) {
-    const uint64_t tiles = narrow_tiles(a);
-    if (tiles > 1 && ws_bytes < narrow_bytes(a))
-        return fail(HX_ERR_DISPATCH_FAILED, "scan workspace of %llu bytes is too small", (unsigned long long)ws_bytes);
-    if (a.exclusive)
-        return a.reverse ? launch_narrow_dir<T, Op, true, true>(p, tiles, ws, stream)
-                         : launch_narrow_dir<T, Op, true, false>(p, tiles, ws, stream);
-    return a.reverse ? launch_narrow_dir<T, Op, false, true>(p, tiles, ws, stream)
-                     : launch_narrow_dir<T, Op, false, false>(p, tiles, ws, stream);
-}
-
-// Row-tile column scans (col_rowtile_*): see the kernels' comment.
+// Row-tile column scans (col_rowtile_lookback_kernel): dense matrices of at
+// most kRowTileMaxCols columns.  A look-back round covers 512 / C
+// predecessors; wider matrices take strips.
+constexpr uint64_t kRowTileMaxCols = 24;
 bool rowtile_column_scan(const ScanArgs &a) {
     const uint64_t c = a.lines;
     const uintptr_t ibase = (uintptr_t)a.in + 4u * a.in_offset; // every element type is 4 bytes
     const uintptr_t obase = (uintptr_t)a.out + 4u * a.out_offset;
-    return c >= 2 && c < kSinglePassMinLines && !narrow_column_scan(a) && a.in_line_stride == 1 &&
-           a.out_line_stride == 1 && a.in_elem_stride == (int64_t)c && a.out_elem_stride == (int64_t)c &&
-           ibase % 4 == 0 && obase % 4 == 0;
-}
-
-// Row-tile scans of more than one tile and at most kRowTileLbMaxCols columns
-// look back (col_rowtile_lookback_kernel) instead of taking three passes:
-// a look-back round covers 512 / C predecessors, and with fewer the chain of
-// tiles falls behind.
-constexpr uint64_t kRowTileLbMaxCols = 24;
-bool rowtile_single_pass(const ScanArgs &a) {
-    return a.lines <= kRowTileLbMaxCols && row_tile_shape(a.lines, a.len).tiles > 1;
-}
-
-uint64_t rowtile_bytes(const ScanArgs &a) {
-    const RowTileShape s = row_tile_shape(a.lines, a.len);
-    if (s.tiles <= 1) return 0;
-    return s.tiles * a.lines * (a.dtype == HX_DTYPE_F32 ? 8u : 4u);
-}
-
-template <typename T, typename Op, bool EXCL, bool REV>
-hx_status launch_rowtile_dir(const ScanParams &p, const RowTileShape &s, void *ws, hipStream_t stream) {
-    using A = typename ColAcc<T>::type;
-    if (s.tiles > 0x7FFFFFFFull) return fail(HX_ERR_DISPATCH_FAILED, "column scan exceeds the grid range");
-    const dim3 grid((uint32_t)s.tiles), block(kRowTileThreads);
-    A *totals = (A *)ws;
-    if (s.tiles > 1) {
-        hipLaunchKernelGGL((col_rowtile_totals_kernel<T, Op, REV>), grid, block, 0, stream, p, s, totals);
-        HX_TRY(check_launch("col_rowtile_totals_kernel"));
-        hipLaunchKernelGGL((col_narrow_carry_kernel<A, Op>), dim3(s.C), dim3(kNarrowCarryThreads), 0, stream, totals,
-                           (uint64_t)1, s.tiles, s.tiles);
-        HX_TRY(check_launch("col_narrow_carry_kernel"));
-        hipLaunchKernelGGL((col_rowtile_scan_kernel<T, Op, EXCL, REV, true>), grid, block, 0, stream, p, s,
-                           (const A *)totals);
-    } else {
-        hipLaunchKernelGGL((col_rowtile_scan_kernel<T, Op, EXCL, REV, false>), grid, block, 0, stream, p, s,
-                           (const A *)totals);
-    }
-    return check_launch("col_rowtile_scan_kernel");
+    return c >= 2 && c <= kRowTileMaxCols && a.in_line_stride == 1 && a.out_line_stride == 1 &&
+           a.in_elem_stride == (int64_t)c && a.out_elem_stride == (int64_t)c && ibase % 4 == 0 && obase % 4 == 0;
 }
 
 uint64_t rowtile_lb_bytes(const ScanArgs &a) {
@@ -2648,16 +2441,140 @@ hx_status launch_rowtile_lb(const ScanArgs &a, ScanParams p, void *ws, uint64_t 
     return r;
 }
 
+// Strip column scans (col_strip_kernel): lines adjacent in memory in both
+// operands, any row pitch.
+//
+// Width: 64 lines, 32 for matrices of at most 32, and for those below 64
+// unless they are large integer ones (u32 / f32, us, 64 and 32 lines wide:
+// [100000, 33] 15.7 / 19.6 and 14.2 / 17.4; [1000003, 48] 73 / 98 and 83 / 92).
+//
+// Rows per lane: 16, and 8 where the matrix is small and its chains stay
+// short (u32, us, 8 / 16 rows: [510, 659] 5.2 / 6.4, [16384, 512] 12.8 / 14.5,
+// [8192, 2048] 26.5 / 28.2, but [100000, 64] 17.5 / 15.5) and where many strips
+// share lines (below).
+constexpr uint64_t kStripSmallElems = 1ull << 24;
+constexpr uint64_t kStripSmallLen = 1ull << 16;
+// Stores of whole lines that go through the L2 all the same: sizes from
+// kStripSmallElems to this, several strips.  u32, us, through the L2 against
+// non-temporal: [65536, 1024] 91 / 102, [16384, 4096] 86 / 101, but [4096,
+// 1024] 8.8 / 8.3, [131072, 1024] 212 / 201 and one strip, [2^20, 64], 88 / 85.
+constexpr uint64_t kStripCachedElems = 1ull << 26;
+// Where strips share lines: chunks dealt to XCDs, if there are enough of
+// them to fill the eight evenly, else strips.  u32, rows / chunks / strips,
+// us: [40000, 1001] 82 / 66 / 75, [100000, 333] 71 / 56 / 83, [12000, 3001]
+// (27 chunks) 68.5 / 63.0 / 62.2, [3782, 5485] (9 chunks) 36.2 / 43.9 / 30.6.
+constexpr uint64_t kStripDealChunks = 32;
+constexpr uint64_t kStripDealStrips = 16;
+// Two blocks on a CU for dealt chunks (by their LDS): with three, the 32 CUs'
+// outputs push half-written lines out of the XCD's 4 MB L2.  With many strips
+// to a chunk, half the rows per block do the same again.  u32, three blocks
+// of 16 rows / two of 16 / two of 8, us: [70000, 2001] 350 / 274 / 224, [140000,
+// 1001] 355 / 270 / 210, [300000, 500] 350 / 256 / 226, [500000, 257] 274 / 217 /
+// 225 (col_lookback_kernel 260, 247, 258, 356).  f32 needs twice the strips:
+// [140000, 1001] - / 249 / 231, [300000, 500] - / 237 / 255.
+constexpr uint32_t kStripDealLds = 54 * 1024;
+constexpr uint64_t kStripDealManyInt = 8, kStripDealManyF32 = 16;
+
+struct StripShape {
+    int W = 64, steps = 16;
+    StripParams sp{};
+    uint64_t blocks = 0;
+    uint32_t lds = 0; // dynamic LDS, for the blocks per CU alone
+};
+
+StripShape strip_shape(const ScanArgs &a) {
+    StripShape s;
+    const uint64_t n = a.len * a.lines;
+    const bool f32 = a.dtype == HX_DTYPE_F32;
+    s.W = a.lines <= 32 || (a.lines < 64 && (f32 || n <= kStripSmallElems)) ? 32 : 64;
+    // The lines are shared out evenly, in whole 16-byte vectors, so that no
+    // strip is left with a few lines (and a block with a few lanes).
+    const uint64_t strips = ceil_div(a.lines, (uint64_t)s.W);
+    s.sp.width = (uint32_t)(ceil_div(ceil_div(a.lines, strips), 4) * 4);
+    s.sp.groups = (uint32_t)ceil_div(a.lines, (uint64_t)s.sp.width);
+    s.sp.lpad = (uint64_t)s.sp.groups * s.W;
+    auto cut = [&](int steps) {
+        s.steps = steps;
+        s.sp.chunks = ceil_div(a.len, steps == 8 ? (s.W == 32 ? StripGeom<32, 8>::kRows : StripGeom<64, 8>::kRows)
+                                                 : (s.W == 32 ? StripGeom<32, 16>::kRows : StripGeom<64, 16>::kRows));
+    };
+    cut(n <= kStripSmallElems && a.len <= kStripSmallLen ? 8 : 16);
+    const bool lines128 = whole_line_rows(a) && s.sp.width % 32 == 0;
+    s.sp.cached = !lines128 || (s.sp.groups > 1 && n > kStripSmallElems && n <= kStripCachedElems) ? 1u : 0u;
+    s.sp.deal = kDealRows;
+    if (!lines128 && s.sp.groups > 1) {
+        if (s.sp.chunks >= kStripDealChunks) {
+            s.sp.deal = kDealChunks;
+            s.lds = kStripDealLds;
+            if (s.sp.groups >= (f32 ? kStripDealManyF32 : kStripDealManyInt)) cut(8);
+        } else if (s.sp.groups >= kStripDealStrips) {
+            s.sp.deal = kDealStrips;
+        }
+    }
+    switch (s.sp.deal) {
+    case kDealChunks: s.blocks = ceil_div(s.sp.chunks, (uint64_t)kXcds) * kXcds * s.sp.groups; break;
+    case kDealStrips: s.blocks = s.sp.chunks * ceil_div((uint64_t)s.sp.groups, (uint64_t)kXcds) * kXcds; break;
+    default: s.blocks = s.sp.chunks * s.sp.groups; break;
+    }
+    return s;
+}
+
+bool strip_column_scan(const ScanArgs &a) {
+    if (a.small_workspace || !column_mode(a) || a.in_line_stride != 1 || a.out_line_stride != 1) return false;
+    if (rowtile_column_scan(a) || column_short_lines(a)) return false;
+    if (column_wide(a) || a.lines >= (1ull << 31)) return false;
+    return strip_shape(a).blocks * (kStripWaves * kWave) <= 0xFFFFFFFFull;
+}
+
+uint64_t strip_bytes(const ScanArgs &a) {
+    const StripShape s = strip_shape(a);
+    return kLookbackOffset + s.sp.chunks * s.sp.lpad * (a.dtype == HX_DTYPE_F32 ? 16u : 8u);
+}
+
+template <typename T, typename Op, typename Status, int W, int STEPS>
+hx_status launch_strip_dir(const ScanParams &p, const StripShape &s, const Status &st, bool excl, bool rev,
+                           hipStream_t stream) {
+    const dim3 grid((uint32_t)s.blocks), block(kStripWaves * kWave);
+    if (excl && rev)
+        hipLaunchKernelGGL((col_strip_kernel<T, Op, Status, W, STEPS, true, true>), grid, block, s.lds, stream, p, s.sp,
+                           st);
+    else if (excl)
+        hipLaunchKernelGGL((col_strip_kernel<T, Op, Status, W, STEPS, true, false>), grid, block, s.lds, stream, p,
+                           s.sp, st);
+    else if (rev)
+        hipLaunchKernelGGL((col_strip_kernel<T, Op, Status, W, STEPS, false, true>), grid, block, s.lds, stream, p,
+                           s.sp, st);
+    else
+        hipLaunchKernelGGL((col_strip_kernel<T, Op, Status, W, STEPS, false, false>), grid, block, s.lds, stream, p,
+                           s.sp, st);
+    return check_launch("col_strip_kernel");
+}
+
+template <typename T, typename Op, typename Status>
+hx_status launch_strip_shaped(const ScanParams &p, const StripShape &s, const Status &st, bool excl, bool rev,
+                              hipStream_t stream) {
+    if (s.W == 32)
+        return s.steps == 8 ? launch_strip_dir<T, Op, Status, 32, 8>(p, s, st, excl, rev, stream)
+                            : launch_strip_dir<T, Op, Status, 32, 16>(p, s, st, excl, rev, stream);
+    return s.steps == 8 ? launch_strip_dir<T, Op, Status, 64, 8>(p, s, st, excl, rev, stream)
+                        : launch_strip_dir<T, Op, Status, 64, 16>(p, s, st, excl, rev, stream);
+}
+
 template <typename T, typename Op>
-hx_status launch_rowtile(const ScanArgs &a, const ScanParams &p, void *ws, uint64_t ws_bytes, hipStream_t stream) {
-    const RowTileShape s = row_tile_shape(a.lines, a.len);
-    if (s.tiles > 1 && ws_bytes < rowtile_bytes(a))
+hx_status launch_strip(const ScanArgs &a, ScanParams p, void *ws, uint64_t ws_bytes, LookbackState &lb,
+                       hipStream_t stream) {
+    const StripShape s = strip_shape(a);
+    if (ws_bytes < strip_bytes(a))
         return fail(HX_ERR_DISPATCH_FAILED, "scan workspace of %llu bytes is too small", (unsigned long long)ws_bytes);
-    if (a.exclusive)
-        return a.reverse ? launch_rowtile_dir<T, Op, true, true>(p, s, ws, stream)
-                         : launch_rowtile_dir<T, Op, true, false>(p, s, ws, stream);
-    return a.reverse ? launch_rowtile_dir<T, Op, false, true>(p, s, ws, stream)
-                     : launch_rowtile_dir<T, Op, false, false>(p, s, ws, stream);
+    HX_TRY(next_lookback_launch(lb, ws, ws_bytes, stream, &p.tag));
+    uint64_t *words = (uint64_t *)((char *)ws + kLookbackOffset);
+    hx_status r;
+    if constexpr (std::is_same<T, float>::value)
+        r = launch_strip_shaped<T, Op>(p, s, F64QuadDense{words}, a.exclusive, a.reverse, stream);
+    else
+        r = launch_strip_shaped<T, Op>(p, s, PackedStatus{words}, a.exclusive, a.reverse, stream);
+    if (r == HX_OK) commit_lookback_launch(lb);
+    return r;
 }
 
 // 16-byte scans of lines longer than one tile whose outputs start off a
@@ -2685,8 +2602,8 @@ uint32_t scan_out_head(const ScanArgs &a) {
 
 uint64_t scan_bytes(const ScanArgs &a) {
     if (short_line_scan(a)) return 0;
-    if (narrow_column_scan(a)) return narrow_bytes(a);
-    if (rowtile_column_scan(a)) return rowtile_single_pass(a) ? rowtile_lb_bytes(a) : rowtile_bytes(a);
+    if (rowtile_column_scan(a)) return rowtile_lb_bytes(a);
+    if (strip_column_scan(a)) return strip_bytes(a);
     if (column_mode(a) && column_single_pass(a)) {
         const ColLbShape c = col_lb_shape(a);
         return kLookbackOffset + c.chunks * c.lpad * (a.dtype == HX_DTYPE_F32 ? 16u : 8u);
@@ -2697,6 +2614,24 @@ uint64_t scan_bytes(const ScanArgs &a) {
     // Lines of one tile never look back and publish no status.
     if (tpl <= 1) return kLookbackOffset;
     return kLookbackOffset + status_bytes(tpl * a.lines) + status_bytes(ceil_div(tpl, kSuper) * a.lines);
+}
+
+// What a fixed workspace must hold for the scan to be taken by a caller that
+// cannot allocate (hx_scan_noalloc).  For strips the requirement is fixed by
+// the matrix alone, whatever the chunks they are cut into: one status a line
+// per 240 rows from 256 lines up; below, one word a line per tile of 32768
+// elements (32, 64 and 128 dense lines) or of whole rows up to 16384, or the
+// chunk totals of padded rows.  Strips that need more than that, near the
+// limit, run chunked instead (small_workspace).
+uint64_t fixed_workspace_bytes(const ScanArgs &a) {
+    if (!strip_column_scan(a)) return scan_bytes(a);
+    const uint64_t word = a.dtype == HX_DTYPE_F32 ? 8u : 4u;
+    if (a.lines >= kSinglePassMinLines)
+        return kLookbackOffset + ceil_div(a.len, kColTileRows) * ceil_div(a.lines, 256) * 256 * 2 * word;
+    if (a.in_elem_stride != (int64_t)a.lines || a.out_elem_stride != (int64_t)a.lines) return column_bytes(a);
+    const bool pow2 = a.lines >= 32 && (a.lines & (a.lines - 1)) == 0;
+    const uint64_t tiles = pow2 ? ceil_div(a.len * a.lines, 32768) : row_tile_shape(a.lines, a.len).tiles;
+    return tiles <= 1 ? 0 : tiles * a.lines * word;
 }
 
 template <typename T, typename Op>
@@ -2720,10 +2655,8 @@ hx_status launch_op(const ScanArgs &a, void *ws, uint64_t ws_bytes, LookbackStat
     if (a.lines == 0 || a.len == 0) return HX_OK;
 
     if (short_line_scan(a)) return launch_short<T, Op>(a, stream);
-    if (narrow_column_scan(a)) return launch_narrow<T, Op>(a, p, ws, ws_bytes, stream);
-    if (rowtile_column_scan(a))
-        return rowtile_single_pass(a) ? launch_rowtile_lb<T, Op>(a, p, ws, ws_bytes, lb, stream)
-                                      : launch_rowtile<T, Op>(a, p, ws, ws_bytes, stream);
+    if (rowtile_column_scan(a)) return launch_rowtile_lb<T, Op>(a, p, ws, ws_bytes, lb, stream);
+    if (strip_column_scan(a)) return launch_strip<T, Op>(a, p, ws, ws_bytes, lb, stream);
     if (column_mode(a) && column_single_pass(a)) {
         const ColLbShape cs = col_lb_shape(a);
         if (cs.groups * cs.chunks > 0x7FFFFFFFull)
@@ -2788,10 +2721,11 @@ hx_status launch_op(const ScanArgs &a, void *ws, uint64_t ws_bytes, LookbackStat
 } // namespace
 
 uint64_t scan_workspace_bytes(const ScanArgs &a) { return scan_bytes(a); }
+uint64_t scan_fixed_workspace_bytes(const ScanArgs &a) { return fixed_workspace_bytes(a); }
 
 bool scan_uses_lookback(const ScanArgs &a) {
-    if (rowtile_column_scan(a)) return rowtile_single_pass(a);
-    if (short_line_scan(a) || narrow_column_scan(a)) return false;
+    if (short_line_scan(a)) return false;
+    if (rowtile_column_scan(a) || strip_column_scan(a)) return true;
     return !column_mode(a) || column_single_pass(a);
 }
 
