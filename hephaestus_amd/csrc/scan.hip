@@ -6,8 +6,9 @@
 // re-reads and re-writes the output (core accelerator/scan.rs:56-155).  A 1-D
 // scan of 2^28 elements therefore runs on one CU.  Here every line is cut
 // into tiles that all CUs process in a single pass (32768 elements for long
-// lines; a line of up to 32768 elements is one tile of the smallest shape
-// that holds it, see tile_shape):
+// lines, 2048 to 8192 for few lines of middling length; of many lines one of
+// up to 32768 elements is one tile of the smallest shape that holds it, see
+// tile_shape):
 //
 //   * block b scans tile b.  The tile is loaded with 16-byte vectors,
 //     wave-striped: step j of wave w holds 256 contiguous elements, lane l
@@ -655,7 +656,12 @@ void scan_tiles_kernel(ScanParams p, Status st, Status st1) {
             if (lane == 0) st.publish_tile(tile, p.tag, kAggregate, agg);
             KnownAgg<C> hook{agg};
             excl = lookback<T, Op, Status, VEC, REV, NT, STEPS, WAVES, HEAD>(p, st, st1, tile, line, tin, hook);
-            if (lane == 0) st.publish_tile(tile, p.tag, kPrefix, Op::combine(excl, agg));
+            // A line of one superblock needs no prefixes: every tile folds
+            // all of its predecessors' aggregates in one poll, always the same
+            // way, so f32 results are reproducible bit for bit (as they are
+            // for lines of one tile).
+            if (lane == 0 && p.tiles_per_line > kSuper)
+                st.publish_tile(tile, p.tag, kPrefix, Op::combine(excl, agg));
         }
         if (lane == 0 && tin % kSuper == kSuper - 1 && tin + 1 < p.tiles_per_line)
             st1.publish(line * p.supers_per_line + tin / kSuper, p.tag, kPrefix, Op::combine(excl, agg));
@@ -2257,8 +2263,8 @@ hx_status launch_column(const ScanParams &p, const ColShape &s, bool rev, void *
 // 16-byte f64 slot at its start).
 uint64_t status_bytes(uint64_t entries) { return entries * kTileStatusBytes; }
 
-// Tile shapes (waves x 16-byte steps per lane).  A line up to 32768
-// elements is one tile: the smallest shape that holds it, so a block never
+// Tile shapes (waves x 16-byte steps per lane).  Of many lines, one up to
+// 32768 elements is one tile: the smallest shape that holds it, so a block never
 // carries idle waves and a row-wise scan needs no look-back.  Longer lines
 // take 8 x 16 tiles chained by the look-back.  Measured on 2^28 u32 (f32)
 // inclusive scans as 65536 x 4096: 1316 us (2329) with 8 x 16 tiles, whose
@@ -2274,7 +2280,26 @@ struct TileShape {
 // f32 lines took 12 x 16 tiles (one block per CU) before f32 tiles fit in
 // 128 VGPRs; 8 x 16 at two blocks per CU: 2^30 f32 1373.1 -> 1315.6 us.
 constexpr int kLongWaves = 8, kLongSteps = 16;
-inline TileShape tile_shape(uint64_t len) {
+// Few lines of more than 2048 elements leave most of the chip idle in tiles
+// that large: a block moves its 128 KiB at one CU's rate, and 2^20 elements
+// are 32 blocks.  Fewer than 256 lines take smaller tiles and chain them,
+// while the tiles number about four or five a CU: 2048 elements up to 2^17,
+// 4096 up to 2^22, 8192 up to kMid8192Elems (2^23 where the outputs do not
+// start on a 128-byte line: the larger tiles then run on the output's grid,
+// scan_out_head).  u32 inclusive (f32), us, one size of tile for all -> now:
+// 10^5 elements 7.4 (8.4) -> 4.0 (4.1), 10^6 7.2 (7.9) -> 5.1 (5.9), 3 * 10^6
+// 9.1 (9.5) -> 6.4 (7.2), 10^7 15.4 (14.9) -> 14.5 (13.8); 16 * 10^6 in 8192s 26.8
+// against 20.4.
+constexpr uint64_t kMidMaxLines = 255;
+constexpr uint64_t kMid2048Elems = 1ull << 17, kMid4096Elems = 1ull << 22, kMid8192Elems = 10ull << 20;
+inline TileShape tile_shape(const ScanArgs &a) {
+    const uint64_t len = a.len, n = a.len * a.lines;
+    if (len > 2048 && a.lines <= kMidMaxLines && a.in_elem_stride == 1 && a.out_elem_stride == 1) {
+        const bool grid = ((uintptr_t)a.out + 4u * a.out_offset + (a.reverse ? 4u * len : 0u)) % 128 == 0;
+        if (n <= kMid2048Elems) return {2, 4};
+        if (n <= kMid4096Elems) return {4, 4};
+        if (len > 4096 && n <= (grid ? kMid8192Elems : 1ull << 23)) return {4, 8};
+    }
     if (len <= 256) return {1, 1};
     if (len <= 512) return {1, 2};
     if (len <= 1024) return {2, 2};
@@ -2285,6 +2310,7 @@ inline TileShape tile_shape(uint64_t len) {
     if (len <= 32768) return {kWaves, kSteps};
     return TileShape{kLongWaves, kLongSteps};
 }
+bool long_tiles(const TileShape &s) { return s.waves == kLongWaves && s.steps == kLongSteps; }
 
 // A launch's work-items (blocks x block size) must stay below 2^32, so many
 // short lines (2^26 lines of at most 512 elements, 2^24 of at most 8192)
@@ -2590,7 +2616,7 @@ hx_status launch_strip(const ScanArgs &a, ScanParams p, void *ws, uint64_t ws_by
 // cost nothing measurable (input offset 1, output aligned: 333 us).
 constexpr uint64_t kOutGrid = 32; // elements: 128 bytes
 uint32_t scan_out_head(const ScanArgs &a) {
-    if (a.len <= 32768 || a.in_elem_stride != 1 || a.out_elem_stride != 1) return 0;
+    if (a.len <= 32768 || a.in_elem_stride != 1 || a.out_elem_stride != 1 || !long_tiles(tile_shape(a))) return 0;
     if (a.lines > 1 && a.out_line_stride % (int64_t)kOutGrid != 0) return 0;
     const uintptr_t ibase = (uintptr_t)a.in + 4u * a.in_offset; // every element type is 4 bytes
     const uintptr_t obase = (uintptr_t)a.out + 4u * a.out_offset;
@@ -2610,7 +2636,7 @@ uint64_t scan_bytes(const ScanArgs &a) {
     }
     if (column_mode(a)) return column_bytes(a);
     const uint64_t vlen = a.len + scan_out_head(a);
-    const uint64_t tpl = ceil_div(vlen, tile_shape(vlen).elems());
+    const uint64_t tpl = ceil_div(vlen, tile_shape(a).elems());
     // Lines of one tile never look back and publish no status.
     if (tpl <= 1) return kLookbackOffset;
     return kLookbackOffset + status_bytes(tpl * a.lines) + status_bytes(ceil_div(tpl, kSuper) * a.lines);
@@ -2641,7 +2667,7 @@ hx_status launch_op(const ScanArgs &a, void *ws, uint64_t ws_bytes, LookbackStat
     p.out = a.out;
     p.lines = a.lines;
     p.len = a.len;
-    const TileShape shape = tile_shape(a.len);
+    const TileShape shape = tile_shape(a);
     p.tiles_per_line = ceil_div(a.len, shape.elems());
     p.total_tiles = p.tiles_per_line * a.lines;
     p.supers_per_line = ceil_div(p.tiles_per_line, kSuper);
