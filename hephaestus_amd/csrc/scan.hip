@@ -780,13 +780,15 @@ void scan_tiles_kernel(ScanParams p, Status st, Status st1) {
 //
 // Line starts are tracked with an incremental remainder, no division per
 // element.  f32 lines scan in f32 (a line holds fewer than 256 elements).
-// Tiles of 8 waves x 16 steps with gaps between stores (as the paced
-// integer tiles): 2^28 u32 along lines of 4 / 100 / 255 elements, 357.9 /
-// 355.5 / 365.6 us without gaps, 354.9 / 357.2 / 358.9 with; 8 steps
-// 406.7 / 417.0 / 419.6 (one tile per line took 16 ms at 4 elements).  f32
-// lines at 16 steps spill a few registers under the 128-VGPR cap and still
-// beat 12 steps, which fit (355.3 / 359.1 / 362.6 against 368.9 / 366.8 /
-// 368.4 us) and 8 steps (395.7 / 404.4 / 410.5).
+// Small tiles: no tile waits for another, so a block that holds little lets
+// the CU overlap many blocks' loads, scans and stores, and small operands
+// fill the chip.  4 waves x 2 steps (2048 elements) for small operands and for
+// lines of a few elements, 4 x 4 beyond (short_tiles_small); us, 4 x 2 / 4 x 4
+// / 8 x 16 tiles: f32 [13635, 48] 3.1 / 4.1 / 18.9; u32 [60000, 100] 7.8 / 7.3 /
+// 12.2, [300000, 40] 15.8 / 17.0 / 17.4; f32 [100000, 200] 29.6 / 27.7 / 36.7,
+// [500000, 250] 163 / 165 / 184, [2684354, 100] 341 / 350 / 385, [1052688, 255]
+// 433 / 367 / 384 (the f32 form of 8 x 16 tiles spilled under the 128-VGPR
+// cap; 8 x 4 tiles 382 / 378 at the last two).
 struct ShortParams {
     const void *in;
     void *out;
@@ -2380,25 +2382,36 @@ hx_status launch_tiles(const ScanParams &p, const Status &st, const Status &st1,
 // Short dense lines (scan_short_lines_kernel): fewer than 256 elements per
 // line, lines packed back to back in input and output.
 constexpr uint64_t kShortLineMax = 256;
-constexpr int kShortWaves = 8, kShortSteps = 16;
+constexpr int kShortWaves = 4;
+constexpr uint64_t kShortSmallElems = 1ull << 22;
+constexpr uint64_t kShortFewLen = 48, kShortFewElems = 1ull << 25;
+bool short_tiles_small(const ShortParams &p) {
+    return p.n <= kShortSmallElems || (p.len <= kShortFewLen && p.n <= kShortFewElems);
+}
 bool short_line_scan(const ScanArgs &a) {
     return a.len >= 1 && a.len < kShortLineMax && a.lines >= 2 && a.in_elem_stride == 1 &&
            a.out_elem_stride == 1 && a.in_line_stride == (int64_t)a.len && a.out_line_stride == (int64_t)a.len;
 }
 
-template <typename T, typename Op, bool EXCL, bool REV>
-hx_status launch_short_dir(ShortParams p, hipStream_t stream) {
-    constexpr uint64_t kTile = (uint64_t)kShortWaves * kWave * 4 * kShortSteps;
+template <typename T, typename Op, bool EXCL, bool REV, int STEPS>
+hx_status launch_short_steps(ShortParams p, hipStream_t stream) {
+    constexpr uint64_t kTile = (uint64_t)kShortWaves * kWave * 4 * STEPS;
     const uint64_t tiles = ceil_div(p.n, kTile);
     const uint64_t max_blocks = std::min<uint64_t>(0x7FFFFFFFull, 0xFFFFFFFFull / (kShortWaves * kWave));
     for (uint64_t t0 = 0; t0 < tiles; t0 += max_blocks) {
         p.tile0 = t0;
-        hipLaunchKernelGGL((scan_short_lines_kernel<T, Op, EXCL, REV, kShortSteps, kShortWaves>),
+        hipLaunchKernelGGL((scan_short_lines_kernel<T, Op, EXCL, REV, STEPS, kShortWaves>),
                            dim3((uint32_t)std::min<uint64_t>(max_blocks, tiles - t0)), dim3(kShortWaves * kWave), 0,
                            stream, p);
         HX_TRY(check_launch("scan_short_lines_kernel"));
     }
     return HX_OK;
+}
+
+template <typename T, typename Op, bool EXCL, bool REV>
+hx_status launch_short_dir(const ShortParams &p, hipStream_t stream) {
+    return short_tiles_small(p) ? launch_short_steps<T, Op, EXCL, REV, 2>(p, stream)
+                                : launch_short_steps<T, Op, EXCL, REV, 4>(p, stream);
 }
 
 template <typename T, typename Op>

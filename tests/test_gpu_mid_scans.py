@@ -67,3 +67,23 @@ def test_mid_scan_under_forced_fallbacks(device, oracle, limits, lines, n):
     for g, l in zip(got_f, f):
         ref, ab = oracle.scan_sum(l, exclusive=False, reverse=True)
         assert oracle.check_f32_bound(g, ref, ab, n)[0] == 0
+
+
+# Short dense lines (fewer than 256 elements) run as one flat range in tiles
+# of 2048 elements up to 2^22 (2^25 for lines of at most 48), 4096 beyond:
+# lines that end at, straddle and exceed tile edges, and a partial last tile.
+@pytest.mark.parametrize("exclusive,reverse", [(False, False), (True, True)])
+@pytest.mark.parametrize("dtype", [np.uint32, np.float32])
+@pytest.mark.parametrize("lines,n", [(8, 255), (9, 255), (32, 64), (33, 64), (2048, 1), (683, 3), (41, 100), (16451, 255),
+                                     (87383, 48), (85600, 49), (41944, 100), (699052, 48), (684786, 49)])
+def test_short_line_tiles(device, oracle, lines, n, dtype, exclusive, reverse):
+    x = (oracle.uniform_int(lines * n, seed=n, lo=0, hi=2**32 - 1) if dtype == np.uint32
+         else oracle.uniform_real(lines * n, seed=n, lo=-1.0, hi=1.0))
+    got = run(device, x, lines, exclusive, reverse)
+    x = x.reshape(lines, n)[:, ::-1 if reverse else 1]
+    want = np.add.accumulate(x, axis=1, dtype=np.uint32 if dtype == np.uint32 else np.float64)
+    bound = 2 * max(1, (n - 1).bit_length()) * 2.0**-23 * np.add.accumulate(np.abs(x), axis=1, dtype=np.float64)
+    if exclusive:
+        want, bound = (np.concatenate([np.zeros((lines, 1), a.dtype), a[:, :-1]], axis=1) for a in (want, bound))
+    want, bound = (a[:, ::-1 if reverse else 1] for a in (want, bound))
+    assert np.array_equal(got, want) if dtype == np.uint32 else np.all(np.abs(got - want) <= bound)
