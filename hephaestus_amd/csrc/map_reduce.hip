@@ -77,6 +77,7 @@ struct MapParams {
     uint64_t n;
     uint64_t a_off, b_off; // element offsets (layout offsets)
     RowsGeom g;            // non-flat views: rows of a, form 2 walks b
+    MatrixWalk m;          // kMatrix: rows of a and of b
     // kPairTile: a is contiguous along the rows, (k, i, j) at a_off + k *
     // col_bs + i + j * col_ld; b along the columns, (k, i, j) at b_off + k *
     // row_bs + i * row_ld + j, for matrices k of a batch.
@@ -91,7 +92,10 @@ struct MapParams {
 // 16-byte vector units (both operands' rows contiguous) or of single
 // elements, or (a dot of a transposed matrix with a row-major one) 64 x 64
 // tiles, the transposed operand's tile turned through LDS.
-enum Mode { kFlat = 0, kRowsVec = 1, kRowsScalar = 2, kPairTile = 3 };
+// kMatrix: rows of contiguous elements under one outer dimension in both
+// operands (MatrixWalk).
+enum Mode { kFlat = 0, kRowsVec = 1, kRowsScalar = 2, kPairTile = 3, kMatrix = 4 };
+constexpr int kMatrixUnits = 4; // units in flight per thread of a matrix walk
 // Tile edge of kPairTile and the LDS pitch of its staged tile: column j of
 // the tile at j * 65, so the 16 columns a wave reads at one row fall in
 // distinct banks.
@@ -281,6 +285,22 @@ __device__ __forceinline__ typename MapPolicy<T, M>::Acc map_thread_fold(const M
                 }
             }
         }
+    } else if constexpr (MODE == kMatrix) {
+        const T *a = (const T *)p.a + (int64_t)p.a_off;
+        const T *b = kTwo ? (const T *)p.b + (int64_t)p.b_off : a;
+        walk_matrix<T, kMatrixUnits, kTwo>(p.m, a, b, tid, nthreads, [&](const auto &x, const auto &y, uint32_t shift,
+                                                                         uint32_t) {
+            Acc e0 = P::elem((T)x.x, (T)y.x), e1 = P::elem((T)x.y, (T)y.y);
+            Acc e2 = P::elem((T)x.z, (T)y.z), e3 = P::elem((T)x.w, (T)y.w);
+            if (ballot(shift != 0u) != 0ull) { // some lane's unit ends a row
+                const Acc id = P::identity();
+                e0 = shift > 0u ? id : e0;
+                e1 = shift > 1u ? id : e1;
+                e2 = shift > 2u ? id : e2;
+                e3 = shift > 3u ? id : e3;
+            }
+            acc = P::combine(acc, P::combine(P::combine(e0, e1), P::combine(e2, e3)));
+        });
     } else {
         // Rows (RowsGeom): kWalkers walkers, each stepping kWalkers * nthreads units.
         const RowsGeom &g = p.g;
@@ -404,6 +424,13 @@ hx_status launch_typed(const MapReduceArgs &a, void *ws, uint64_t ws_bytes, Look
                            dim3(kBlock), 0, stream, p);
     } else {
         const RowsView rv = layout_rows_pair(a.a_layout, M == kMapDot ? a.b_layout : a.a_layout);
+        if (is_matrix_walk(rv) && rv.cstride2 == 1) {
+            p.m = matrix_walk(rv, (uint64_t)blocks * kBlock, kMatrixUnits);
+            hipLaunchKernelGGL((map_reduce_kernel<T, M, kMatrix>), dim3(blocks), dim3(kBlock), 0, stream, p);
+            HX_TRY(check_launch("map_reduce_kernel"));
+            commit_lookback_launch(lb);
+            return HX_OK;
+        }
         const bool vec = rv.cstride == 1 && rv.cstride2 == 1 && rv.cols >= 4;
         p.g = rows_geom(rv, vec, (uint64_t)MapWalkers<M == kMapDot>::value * blocks * kBlock);
         if (vec)

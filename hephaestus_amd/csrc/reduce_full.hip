@@ -116,6 +116,7 @@ struct FullParams {
     uint64_t n;
     uint64_t offset; // element offset of the view (flat) / layout offset
     RowsGeom g;      // non-flat views
+    MatrixWalk m;    // kMatrix
     float a, b;
     void *out_value;
     uint32_t *out_index;
@@ -188,13 +189,16 @@ __device__ __forceinline__ typename P::Acc fold4(const V &v, uint64_t e, bool re
     return P::combine(P::combine(a0, a1), P::combine(a2, a3));
 }
 
-// How a view is walked: the flat element range, or rows (RowsGeom) of
-// 16-byte vector units (contiguous rows) or of single elements.
-enum Mode { kFlat = 0, kRowsVec = 1, kRowsScalar = 2 };
+// How a view is walked: the flat element range, the rows of a matrix
+// (MatrixWalk), or rows under more dimensions (RowsGeom) of 16-byte vector
+// units (contiguous rows) or of single elements.
+enum Mode { kFlat = 0, kRowsVec = 1, kRowsScalar = 2, kMatrix = 3 };
+// Units in flight per thread of a matrix walk.
+constexpr int kMatrixUnits = 4;
 // Walkers (units in flight per thread) of the row modes.  A 65536 x 4000
-// slice of 4096-wide f32 rows: 2 walkers 262 us, 4 walkers 170 us (dense:
-// 153 us), with the row tail loaded by unrolled predicated loads (a
-// runtime-indexed tail loop cost 35%).
+// slice of 4096-wide f32 rows (a matrix walk now): 2 walkers 262 us, 4
+// walkers 170 us (dense: 153 us), with the row tail loaded by unrolled
+// predicated loads (a runtime-indexed tail loop cost 35%).
 template <int MODE> struct Walkers { static constexpr int value = 4; };
 
 // Unit of walker `w`: its elements in x[0..count), returned count.
@@ -286,6 +290,23 @@ __device__ __forceinline__ typename P::Acc thread_fold(const FullParams &p, uint
             const uint64_t e = tail0 + tid;
             acc = P::combine(acc, P::lift(prologue<T, AFFINE>(src[e], p.a, p.b), vidx(e)));
         }
+    } else if constexpr (MODE == kMatrix) {
+        const T *src = (const T *)p.base + (int64_t)p.offset;
+        walk_matrix<T, kMatrixUnits, false>(p.m, src, src, tid, nthreads, [&](const auto &x, const auto &, uint32_t shift,
+                                                                              uint32_t i) {
+            Acc a0 = P::lift(prologue<T, AFFINE>((T)x.x, p.a, p.b), i);
+            Acc a1 = P::lift(prologue<T, AFFINE>((T)x.y, p.a, p.b), i + 1u);
+            Acc a2 = P::lift(prologue<T, AFFINE>((T)x.z, p.a, p.b), i + 2u);
+            Acc a3 = P::lift(prologue<T, AFFINE>((T)x.w, p.a, p.b), i + 3u);
+            if (ballot(shift != 0u) != 0ull) { // some lane's unit ends a row
+                const Acc id = P::identity();
+                a0 = shift > 0u ? id : a0;
+                a1 = shift > 1u ? id : a1;
+                a2 = shift > 2u ? id : a2;
+                a3 = shift > 3u ? id : a3;
+            }
+            acc = P::combine(acc, P::combine(P::combine(a0, a1), P::combine(a2, a3)));
+        });
     } else {
         constexpr int W = Walkers<MODE>::value;
         const RowsGeom &g = p.g;
@@ -378,6 +399,15 @@ hx_status launch_typed(const FullReduceArgs &a, void *ws, uint64_t ws_bytes, Loo
         hipLaunchKernelGGL((full_reduce_kernel<T, K, AFFINE, kFlat>), dim3(blocks), dim3(kBlock), 0, stream, p);
     } else {
         const RowsView rv = a.memory_order ? layout_rows_memory_order(a.layout) : layout_rows(a.layout);
+        // The logical index a walker carries is 32 bits; argmax (the only kind
+        // that reads it) takes at most 2^32 - 2 elements, in logical order.
+        if (is_matrix_walk(rv) && !a.memory_order) {
+            p.m = matrix_walk(rv, (uint64_t)blocks * kBlock, kMatrixUnits);
+            hipLaunchKernelGGL((full_reduce_kernel<T, K, AFFINE, kMatrix>), dim3(blocks), dim3(kBlock), 0, stream, p);
+            HX_TRY(check_launch("full_reduce_kernel"));
+            commit_lookback_launch(lb);
+            return HX_OK;
+        }
         const bool vec = rv.cstride == 1 && rv.cols >= 4;
         p.g = rows_geom(rv, vec, (uint64_t)(vec ? Walkers<kRowsVec>::value : Walkers<kRowsScalar>::value) *
                                      blocks * kBlock);
