@@ -497,6 +497,14 @@ __global__ __launch_bounds__(kBlock) void rows_tile_kernel(RowParams p, uint32_t
     }
 }
 
+// First of the V outputs of the lane that `want` falls to.  Where the outputs
+// are no multiple of 4 the last lane moves back to a whole vector: it shares
+// outputs with its neighbour, and both write the same bits.  One output per
+// lane for such matrices: [23542, 573] f32 sum 14.5 us + fold against 10.6.
+template <int V> __device__ __forceinline__ uint64_t cols_first_output(uint64_t want, uint64_t outputs) {
+    return V == 4 && want + 4 > outputs ? outputs - 4 : want;
+}
+
 // Statistics of lines [j0, j1) of the 64*V adjacent outputs from o0 (V per
 // lane) of a column tile, kU lines in flight per lane: V = 4 gives every
 // lane one 16-byte load per line, so each load instruction of a wave covers
@@ -523,7 +531,19 @@ __device__ __forceinline__ void cols_walk(const RowParams &p, uint64_t o0, uint6
 #pragma unroll
             for (int u = 0; u < kU; ++u) visit(x[u], (uint32_t)(j + u));
         }
-        for (; j < j1; ++j) visit(__builtin_nontemporal_load((const Vt *)(base + (int64_t)j * p.col_stride)), (uint32_t)j);
+        // The last lines together as well (past the end: the last one again,
+        // not visited): taken one by one they are a memory round trip each.
+        if (j < j1) {
+            Vt x[kU];
+#pragma unroll
+            for (int u = 0; u < kU; ++u) {
+                const uint64_t l = j + u < j1 ? j + u : j1 - 1;
+                x[u] = __builtin_nontemporal_load((const Vt *)(base + (int64_t)l * p.col_stride));
+            }
+#pragma unroll
+            for (int u = 0; u < kU; ++u)
+                if (j + u < j1) visit(x[u], (uint32_t)(j + u));
+        }
     } else {
         for (; j + kU <= j1; j += kU) {
             T x[kU];
@@ -538,6 +558,10 @@ __device__ __forceinline__ void cols_walk(const RowParams &p, uint64_t o0, uint6
     }
 }
 
+// Statistic planes a flag set keeps (sum or mean, product, max or argmax, min).
+template <int FLAGS> constexpr int kPlanes = ((FLAGS & (F_SUM | F_MEAN)) != 0) + ((FLAGS & F_PROD) != 0) +
+                                             ((FLAGS & (F_ARG | F_MAX)) != 0) + ((FLAGS & F_MIN) != 0);
+
 // Column tiles (the reduced axis is strided, the outputs adjacent: axis-0
 // reduction of a row-major matrix).  A wave owns 64*V adjacent outputs and
 // one chunk of the reduced axis (cols_walk).  Adjacent waves take adjacent
@@ -550,8 +574,9 @@ __global__ __launch_bounds__(kBlock) void cols_tiles_kernel(RowParams p, uint64_
     const uint64_t w = ((uint64_t)blockIdx.x * kBlock + threadIdx.x) / kWave;
     if (w >= groups * nchunks) return;
     const uint64_t g = w % groups, k = w / groups;
-    const uint64_t o0 = (g * kWave + (uint64_t)lane_id()) * V;
-    if (o0 >= p.rows) return;
+    const uint64_t want = (g * kWave + (uint64_t)lane_id()) * V;
+    if (want >= p.rows) return;
+    const uint64_t o0 = cols_first_output<V>(want, p.rows);
     const uint64_t j0 = k * chunk;
     const uint64_t j1 = j0 + chunk < p.cols ? j0 + chunk : p.cols;
     Stats<T, FLAGS> st[V];
@@ -565,43 +590,52 @@ __global__ __launch_bounds__(kBlock) void cols_tiles_kernel(RowParams p, uint64_
     }
 }
 
-// Small column reductions in one launch, with no workspace: a block of
-// kFoldSlices waves per output group, wave s walking slice s of the reduced
-// axis (`chunk` lines), then lane o of wave 0 folding the slices' statistics
-// through LDS in slice order, one component at a time, and writing the
-// outputs.  The order depends only on the shape, so f32 sums are bitwise
-// reproducible.  The split form (column tiles into partial planes, then
-// split_fold_kernel) takes two launches; on a 256 x 256 f32 axis-0 sum that
-// is about 6 us per call, each launch costing a few microseconds of host and
-// device time whatever its size.
-template <typename T, bool AFFINE, int FLAGS, int V>
-__global__ __launch_bounds__(kWave *kFoldSlices) void cols_block_kernel(RowParams p, uint64_t chunk) {
-    __shared__ uint64_t sh[kMaxPlanes * kFoldSlices * kWave];
+// Column reductions in one launch, with no workspace: a block of WAVES waves
+// per group of LANES * V outputs.  LANES lanes make a row of the group and
+// 64 / LANES rows a load instruction, so the axis is cut into WAVES * 64 / LANES
+// slices; the slices of a wave merge with xor shuffles, and a thread per
+// output folds the waves' statistics through LDS in wave order and writes it.
+// The order depends only on the shape, so f32 sums are bitwise reproducible.
+// Adjacent groups run on one XCD: where rows start off the 128-byte grid
+// they share lines (1000 x 50001 f32, 16 lanes: 48 us without, 38 with).
+//
+// The split form (column tiles into partial planes, then split_fold_kernel)
+// takes two launches, 7.7 us whatever its size.  f32 sum, us, split -> block:
+// 256 x 256 4.2 -> 3.7, 1024 x 1024 18.4 -> 4.6 and 1000 x 64 10.9 -> 4.1
+// against the form with 64 lanes of one output and a serial slice per wave,
+// 300 x 4096 7.9 -> 4.0, 34 x 200000 34 -> 6.6, 300 x 200000 73 -> 40,
+// 500 x 500000 221 -> 154.
+template <typename T, bool AFFINE, int FLAGS, int V, int LANES, int WAVES>
+__global__ __launch_bounds__(kWave *WAVES) void cols_block_kernel(RowParams p, uint64_t chunk) {
+    constexpr int kOutputs = LANES * V;
+    static_assert(kOutputs <= kWave * WAVES, "a thread per output");
+    __shared__ uint64_t sh[kPlanes<FLAGS> * WAVES * kOutputs];
     const int lane = lane_id();
     const int s = threadIdx.x / kWave;
-    const uint64_t o0 = ((uint64_t)blockIdx.x * kWave + (uint64_t)lane) * V;
-    const bool live = o0 < p.rows; // V = 4 only when rows % 4 == 0: all four outputs exist
-    const uint64_t j0 = (uint64_t)s * chunk < p.cols ? (uint64_t)s * chunk : p.cols;
+    const int q = lane % LANES;
+    const uint64_t group = xcd_contiguous(blockIdx.x, gridDim.x); // past the last: idle
+    const uint64_t want = (group * LANES + (uint64_t)q) * V;
+    const uint64_t part = (uint64_t)s * (kWave / LANES) + (uint64_t)(lane / LANES);
+    const uint64_t j0 = part * chunk < p.cols ? part * chunk : p.cols;
     const uint64_t j1 = j0 + chunk < p.cols ? j0 + chunk : p.cols;
     Stats<T, FLAGS> st[V];
-    if (live) cols_walk<T, AFFINE, FLAGS, V>(p, o0, j0, j1, st);
-    constexpr uint64_t kPlane = (uint64_t)kFoldSlices * kWave;
+    if (want < p.rows) cols_walk<T, AFFINE, FLAGS, V>(p, cols_first_output<V>(want, p.rows), j0, j1, st);
+    constexpr uint64_t kPlane = (uint64_t)WAVES * kOutputs;
 #pragma unroll
     for (int v = 0; v < V; ++v) {
-        st[v].store_partial(&sh[s * kWave + lane], kPlane);
-        __syncthreads();
-        if (s == 0 && live) {
-            Stats<T, FLAGS> total;
-            for (int q = 0; q < kFoldSlices; ++q) total.merge_partial(&sh[q * kWave + lane], kPlane);
-            total.write(p, o0 + v);
-        }
-        __syncthreads();
+#pragma unroll
+        for (int m = LANES; m < kWave; m <<= 1) st[v].merge_xor(m);
+        if (lane < LANES) st[v].store_partial(&sh[s * kOutputs + q * V + v], kPlane);
     }
+    __syncthreads();
+    // Thread t: component t % V of lane t / V.
+    const uint64_t mine = (group * LANES + threadIdx.x / V) * V;
+    if (threadIdx.x >= kOutputs || mine >= p.rows) return;
+    Stats<T, FLAGS> total;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) total.merge_partial(&sh[w * kOutputs + threadIdx.x], kPlane);
+    total.write(p, cols_first_output<V>(mine, p.rows) + threadIdx.x % V);
 }
-
-// Statistic planes a flag set keeps (sum or mean, product, max or argmax, min).
-template <int FLAGS> constexpr int kPlanes = ((FLAGS & (F_SUM | F_MEAN)) != 0) + ((FLAGS & F_PROD) != 0) +
-                                             ((FLAGS & (F_ARG | F_MAX)) != 0) + ((FLAGS & F_MIN) != 0);
 
 constexpr uint64_t kPeriodMaxCols = 95; // the period form's widest matrix
 
@@ -734,43 +768,57 @@ __global__ __launch_bounds__(kBlock) void rows_split_kernel(RowParams p, uint64_
     if (lane == 0) st.store_partial(partials + k * p.rows + r, (uint64_t)nchunks * p.rows);
 }
 
-// Fold the chunk partials: a block owns 64 outputs (lanes) and kFoldSlices
-// waves; wave s folds its contiguous range of chunks in order, then lane o of
-// wave 0 folds the slice results in slice order.  The order depends only on
+// Fold the chunk partials: a block owns OUTPUTS outputs and cuts the chunks
+// into kFoldSlices * 64 / OUTPUTS contiguous slices, one to every OUTPUTS
+// lanes: 16 outputs, or 64 from kFoldManyOutputs (f32 sum with its tiles, us,
+// 64 / 16: 1779 x 8200 14.8 / 17.2, 10000 x 4099 33.0 / 33.5, 3000 x 2048
+// 10.2 / 9.5, 23542 x 573 19.8 / 16.6, 100000 x 100 28.5 / 16.6).
+// A lane folds its slice in order, kFoldBatch partials loaded together; the
+// wave's slices merge with xor shuffles, and lane o of wave 0 folds the
+// waves' results in wave order.  The order depends only on
 // the chunk count, so f32 sums do not depend on scheduling.
+constexpr uint64_t kFoldManyOutputs = 4096;
+constexpr int kFoldBatch = 8;
 
-template <typename T, int FLAGS>
+template <typename T, int FLAGS, int OUTPUTS>
 __global__ __launch_bounds__(kWave *kFoldSlices) void split_fold_kernel(RowParams p, const uint64_t *partials,
                                                                        uint32_t nchunks) {
-    __shared__ uint64_t sh[kMaxPlanes * kFoldSlices * kWave];
+    constexpr uint32_t kSlices = kFoldSlices * (kWave / OUTPUTS);
+    __shared__ uint64_t sh[kPlanes<FLAGS> * kFoldSlices * OUTPUTS];
     const int lane = lane_id();
-    const int s = threadIdx.x / kWave;
-    const uint64_t o = (uint64_t)blockIdx.x * kWave + lane;
+    const int w = threadIdx.x / kWave;
+    const int q = lane % OUTPUTS;
+    const uint32_t s = (uint32_t)(w * (kWave / OUTPUTS) + lane / OUTPUTS);
+    const uint64_t o = (uint64_t)blockIdx.x * OUTPUTS + q;
     const uint64_t plane = (uint64_t)nchunks * p.rows;
-    const uint32_t per = (nchunks + kFoldSlices - 1) / kFoldSlices;
+    const uint32_t per = (nchunks + kSlices - 1) / kSlices;
     const uint32_t k0 = s * per < nchunks ? s * per : nchunks;
     const uint32_t k1 = k0 + per < nchunks ? k0 + per : nchunks;
     Stats<T, FLAGS> st;
     if (o < p.rows) {
-        // Eight partials loaded together, then merged in chunk order (one
-        // dependent load per chunk left a 3-output fold of 2049 chunks at
-        // 34 us).
-        uint32_t k = k0;
-        for (; k + 8 <= k1; k += 8) {
-            Stats<T, FLAGS> b[8];
+        // One dependent load per chunk left a 3-output fold of 2049 chunks at
+        // 34 us.
+        for (uint32_t k = k0; k < k1; k += kFoldBatch) {
+            Stats<T, FLAGS> b[kFoldBatch];
 #pragma unroll
-            for (int u = 0; u < 8; ++u)
-                b[u] = Stats<T, FLAGS>::from_partial(partials + (uint64_t)(k + u) * p.rows + o, plane);
+            for (uint32_t u = 0; u < kFoldBatch; ++u) {
+                const uint32_t c = k + u < k1 ? k + u : k1 - 1; // past the slice: loaded, not merged
+                b[u] = Stats<T, FLAGS>::from_partial(partials + (uint64_t)c * p.rows + o, plane);
+            }
 #pragma unroll
-            for (int u = 0; u < 8; ++u) st.merge(b[u]);
+            for (uint32_t u = 0; u < kFoldBatch; ++u)
+                if (k + u < k1) st.merge(b[u]);
         }
-        for (; k < k1; ++k) st.merge_partial(partials + (uint64_t)k * p.rows + o, plane);
     }
-    st.store_partial(&sh[s * kWave + lane], (uint64_t)kFoldSlices * kWave);
+#pragma unroll
+    for (int m = OUTPUTS; m < kWave; m <<= 1) st.merge_xor(m);
+    constexpr uint64_t kPlane = (uint64_t)kFoldSlices * OUTPUTS;
+    if (lane < OUTPUTS) st.store_partial(&sh[w * OUTPUTS + q], kPlane);
     __syncthreads();
-    if (s != 0 || o >= p.rows) return;
+    if (threadIdx.x >= OUTPUTS || o >= p.rows) return;
     Stats<T, FLAGS> total;
-    for (int q = 0; q < kFoldSlices; ++q) total.merge_partial(&sh[q * kWave + lane], (uint64_t)kFoldSlices * kWave);
+#pragma unroll
+    for (int k = 0; k < kFoldSlices; ++k) total.merge_partial(&sh[k * OUTPUTS + q], kPlane);
     total.write(p, o);
 }
 
@@ -779,16 +827,40 @@ __global__ __launch_bounds__(kWave *kFoldSlices) void split_fold_kernel(RowParam
 // 128 lines each ran at 6.7 TB/s with the fold; 4096 waves 6.4; 8192 waves
 // 5.0 (a second, mostly idle round of waves).
 constexpr uint64_t kTargetWaves = 2048;
-constexpr uint64_t kMinColChunk = 32;    // lines per column-tile chunk
+// Lines per column-tile chunk, at least; half as many up to kShortCols lines,
+// where 32 leave CUs without a wave (f32 sum, us, 32 -> 16 lines a chunk:
+// 1779 x 1398 9.0 -> 7.7, 3000 x 837 8.6 -> 7.6, 5000 x 506 9.0 -> 7.8;
+// 10000 x 506 9.7 -> 10.7, 30000 x 195 11.0 -> 13.4).
+constexpr uint64_t kMinColChunk = 32;
+constexpr uint64_t kShortCols = 4096;
 constexpr uint64_t kMinRowChunk = 8192;  // elements per split-row chunk
 constexpr uint64_t kRowTargetWaves = 4096; // split rows when fewer than half this many
 
-// Column reductions that would split their axis take one launch
-// (cols_block_kernel) when the matrix is small: at most kBlockFoldLines lines
-// (64 per wave) and kBlockFoldElems elements.
+// Column reductions of more than kMinColChunk lines take one launch
+// (cols_block_kernel) as follows; anything else the column tiles, whose
+// chunks are long enough there.
+// Vectors, at least kWideCols outputs (192 blocks of 256): 64 lanes and 8
+// waves, 1 KiB of a line to a load.  Up to 512 lines always, beyond up to
+// kWideLines if the blocks fill the CUs evenly -- at most one each, or a
+// last round no more than a fifth empty.  f32 sum, us, this / 16 lanes /
+// tiles: 300 x 50001 11 / 17 / 21, 1024 x 65536 43 / 53 / 60, 5000 x 60000
+// 177 / 188 / 189; uneven, 1000 x 200000 135 / 121 / 167.
+// Other vectors: 16 lanes and 16 waves, 256 bytes of a line to a row, up to
+// kBlockFoldLines lines, or four times as many from kBlockManyCols outputs
+// (160 blocks of 64).  f32 sum, us, this / tiles: 1024 x 256 4.3 / 7.9,
+// 1500 x 256 5.8 / 8.0, 2048 x 256 6.4 / 7.6, 2048 x 100 12.7 / 7.8,
+// 2500 x 8192 20 / 19, 2500 x 12000 20 / 26, 5000 x 12000 38 / 44,
+// 5000 x 30000 100 / 97.
+// Strided outputs: a lane per output and a serial slice per wave, up to
+// kBlockFoldLines lines and kBlockFoldElems elements.
 constexpr uint64_t kBlockFoldLines = 64 * kFoldSlices;
 constexpr uint64_t kBlockFoldElems = 1ull << 20;
-
+constexpr uint64_t kBlockManyCols = 160 * 64;
+constexpr uint64_t kWideCols = 192 * 256;
+constexpr uint64_t kWideLines = 8192;
+constexpr uint64_t kCus = 256;
+constexpr int kBlockLanes = 16;
+constexpr int kWideWaves = 8;
 // Axis 0 of a dense row-major matrix with any other column count below 96,
 // more than kBlockFoldLines lines (fewer take the one-launch block form) and
 // row indices within 32 bits: the period form, cols_period_kernel.  From 96
@@ -807,6 +879,8 @@ struct Shape {
     bool period = false; // cols_period_kernel over residues mod P of 1 KiB blocks
     uint32_t P = 1, waves = 0;
     bool block = false; // cols_block_kernel: one launch, no partials
+    int lanes = kWave;  // its lanes per row and waves
+    int block_waves = kFoldSlices;
     bool tile = false;  // rows_tile_kernel: tiles of tile_rows short rows
     uint32_t tile_rows = 0;
     int tile_group = 1; // lanes per row of the tile
@@ -815,6 +889,23 @@ struct Shape {
     uint64_t groups = 0, chunk = 0;
     uint32_t nchunks = 1;
 };
+
+// Whether a column reduction takes cols_block_kernel, and its lanes and waves
+// (s.vec and s.groups, the groups of 64 lanes, are set).
+bool block_columns(const RowParams &p, Shape &s) {
+    if (p.cols <= kMinColChunk) return false;
+    if (!s.vec)
+        return s.groups < kTargetWaves && p.cols <= kBlockFoldLines && p.rows * p.cols <= kBlockFoldElems;
+    if (p.rows >= kWideCols) {
+        const uint64_t rounds = ceil_div(s.groups, kCus);
+        const bool even = rounds == 1 || rounds * kCus * 4 <= s.groups * 5;
+        s.block_waves = kWideWaves;
+        if (p.cols <= 512 || (p.cols <= kWideLines && even)) return true;
+    }
+    s.lanes = kBlockLanes;
+    s.block_waves = kFoldSlices;
+    return p.cols <= (p.rows >= kBlockManyCols ? 4 : 1) * kBlockFoldLines;
+}
 
 // Lanes per row: the largest group that still gives each lane at least
 // three 16-byte vectors of the row, except that a wave per row pays for a
@@ -874,12 +965,20 @@ Shape plan_shape(const RowParams &p, bool cols_layout) {
     }
     if (cols_layout) {
         // 16-byte vectors at 4-byte alignment (Vec4A4): any line start.
-        s.vec = p.row_stride == 1 && p.rows % 4 == 0 && base % 4 == 0;
+        s.vec = p.row_stride == 1 && p.rows >= 4 && base % 4 == 0;
         s.V = s.vec ? 4 : 1;
         s.groups = ceil_div(p.rows, (uint64_t)kWave * s.V);
+        if (block_columns(p, s)) {
+            s.block = true;
+            s.groups = ceil_div(p.rows, (uint64_t)s.lanes * s.V);
+            s.chunk = ceil_div(p.cols, (uint64_t)(s.block_waves * (kWave / s.lanes)));
+            return s;
+        }
         if (s.groups < kTargetWaves) {
-            k = ceil_div(kTargetWaves, s.groups);
-            const uint64_t kmax = ceil_div(p.cols, kMinColChunk);
+            // No more than kTargetWaves: a few beyond leave some CUs a block
+            // more than the others (20000 x 12000 f32 sum 180 -> 153 us.  Above half of it two chunks all the same.
+            k = s.groups <= kTargetWaves / 2 ? kTargetWaves / s.groups : 2;
+            const uint64_t kmax = ceil_div(p.cols, p.cols <= kShortCols ? kMinColChunk / 2 : kMinColChunk);
             if (k > kmax) k = kmax;
         }
     } else {
@@ -898,12 +997,6 @@ Shape plan_shape(const RowParams &p, bool cols_layout) {
         }
     }
     if (k < 1) k = 1;
-    if (cols_layout && k > 1 && p.cols <= kBlockFoldLines && p.rows * p.cols <= kBlockFoldElems) {
-        s.block = true;
-        s.chunk = ceil_div(p.cols, (uint64_t)kFoldSlices);
-        s.nchunks = 1;
-        return s;
-    }
     if (k > 1) {
         uint64_t chunk = ceil_div(p.cols, k);
         if (!cols_layout) chunk = ceil_div(chunk, 256) * 256; // whole 1 KiB wave loads per chunk
@@ -941,11 +1034,17 @@ hx_status launch_rows_typed(const RowParams &p, bool cols_layout, void *ws, uint
         HX_TRY(check_launch("cols_period_kernel"));
     } else if (s.block) {
         if (s.groups > 0x7FFFFFFFull) return fail(HX_ERR_DISPATCH_FAILED, "axis reduction exceeds the grid range");
-        const dim3 grid((uint32_t)s.groups), block(kWave * kFoldSlices);
-        if (s.vec)
-            hipLaunchKernelGGL((cols_block_kernel<T, AFFINE, FLAGS, 4>), grid, block, 0, stream, p, s.chunk);
+        // Whole sets of 8 blocks, so that adjacent groups can share an XCD.
+        const dim3 grid((uint32_t)(s.groups >= 16 ? ceil_div(s.groups, 8) * 8 : s.groups)), block(kWave * s.block_waves);
+        if (!s.vec)
+            hipLaunchKernelGGL((cols_block_kernel<T, AFFINE, FLAGS, 1, kWave, kFoldSlices>), grid, block, 0, stream, p,
+                               s.chunk);
+        else if (s.lanes == kWave)
+            hipLaunchKernelGGL((cols_block_kernel<T, AFFINE, FLAGS, 4, kWave, kWideWaves>), grid, block, 0, stream, p,
+                               s.chunk);
         else
-            hipLaunchKernelGGL((cols_block_kernel<T, AFFINE, FLAGS, 1>), grid, block, 0, stream, p, s.chunk);
+            hipLaunchKernelGGL((cols_block_kernel<T, AFFINE, FLAGS, 4, kBlockLanes, kFoldSlices>), grid, block, 0, stream,
+                               p, s.chunk);
         return check_launch("cols_block_kernel");
     } else if (cols_layout) {
         const uint64_t waves = s.groups * s.nchunks;
@@ -1026,8 +1125,13 @@ hx_status launch_rows_typed(const RowParams &p, bool cols_layout, void *ws, uint
         return HX_OK;
     }
     if (!split) return HX_OK;
-    hipLaunchKernelGGL((split_fold_kernel<T, FLAGS>), dim3((uint32_t)ceil_div(p.rows, kWave)),
-                       dim3(kWave * kFoldSlices), 0, stream, p, (const uint64_t *)partials, s.nchunks);
+    const dim3 fold_block(kWave * kFoldSlices);
+    if (p.rows >= kFoldManyOutputs)
+        hipLaunchKernelGGL((split_fold_kernel<T, FLAGS, 64>), dim3((uint32_t)ceil_div(p.rows, 64)), fold_block, 0, stream,
+                           p, (const uint64_t *)partials, s.nchunks);
+    else
+        hipLaunchKernelGGL((split_fold_kernel<T, FLAGS, 16>), dim3((uint32_t)ceil_div(p.rows, 16)), fold_block, 0, stream,
+                           p, (const uint64_t *)partials, s.nchunks);
     return check_launch("split_fold_kernel");
 }
 
