@@ -24,6 +24,11 @@ constexpr uint32_t kMaxBlocks = 2048;
 constexpr int kTileWaves = 8;
 constexpr int kTileSteps = 32;
 constexpr uint64_t kTileBytes = (uint64_t)kTileWaves * kWave * 16 * kTileSteps;
+// Fewer bytes go to copy_vec_kernel whole: 256 KiB tiles leave CUs idle there
+// and the remainder costs a second launch.  us, tiles (and remainder) / vectors:
+// 262144 bytes 5.5 / 3.6, 266052 7.7 / 3.6, 8 MiB 6.1 / 3.6, 16 MiB 6.4 / 4.8,
+// 32 MiB 12.2 / 10.7, 64 MiB 18.6 / 21.7, 512 MiB 166 / 197.
+constexpr uint64_t kTilesFrom = 48ull << 20;
 
 __global__ __launch_bounds__(kTileWaves * kWave) void copy_tiles_kernel(const char *src, char *dst) {
     const uint64_t base = (uint64_t)xcd_contiguous(blockIdx.x, gridDim.x) * kTileBytes;
@@ -123,7 +128,7 @@ hx_status launch_copy(const void *src, void *dst, uint64_t bytes, hipStream_t st
     if (bytes == 0) return ok();
     const bool aligned = (((uintptr_t)src | (uintptr_t)dst) & 3u) == 0; // 16-byte vectors at 4-byte alignment
     if (aligned) {
-        const uint64_t tiles = bytes / kTileBytes;
+        const uint64_t tiles = bytes < kTilesFrom ? 0 : bytes / kTileBytes;
         if (tiles >= 0x80000000ull)
             return fail(HX_ERR_DISPATCH_FAILED, "copy of %llu bytes exceeds the grid range",
                         (unsigned long long)bytes);
