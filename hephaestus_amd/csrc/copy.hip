@@ -91,6 +91,23 @@ __global__ __launch_bounds__(kScanShapeWaves * kWave) void copy_scan_shape_kerne
     for (int j = 0; j < kScanShapeSteps; ++j) stream_store(v[j], orsrc, lane_off + (uint32_t)j * (kWave * 16));
 }
 
+// Small read-back: `bytes` (4-byte words where the addresses allow) to pinned
+// host memory, then `sequence` to the slot's flag once they are visible to the
+// host.  One block; bytes = 0 only sets the flag.
+constexpr int kReadBackBlock = 64;
+__global__ __launch_bounds__(kReadBackBlock) void read_back_kernel(const uint8_t *src, uint8_t *dst, uint32_t bytes,
+                                                                  uint64_t *flag, uint64_t sequence) {
+    uint32_t done = 0;
+    if (((uintptr_t)src & 3u) == 0) {
+        for (uint32_t i = threadIdx.x; i < bytes / 4; i += kReadBackBlock) ((uint32_t *)dst)[i] = ((const uint32_t *)src)[i];
+        done = bytes & ~3u;
+    }
+    for (uint32_t i = done + threadIdx.x; i < bytes; i += kReadBackBlock) dst[i] = src[i];
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x == 0) __hip_atomic_store(flag, sequence, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // Zero `count` 64-bit words.  Used where status words must be cleared on a
 // stream that a caller may capture into a HIP graph (a kernel node replays
 // correctly where a captured memset node may not).
@@ -108,6 +125,13 @@ hx_status launch_clear_words(void *words, uint64_t count, hipStream_t stream) {
     hipLaunchKernelGGL(clear_words_kernel, dim3((uint32_t)blocks), dim3(kBlock), 0, stream, (uint64_t *)words,
                        count);
     return check_launch("clear_words_kernel");
+}
+
+hx_status launch_read_back(const void *src, void *dst, uint32_t bytes, uint64_t *flag, uint64_t sequence,
+                           hipStream_t stream) {
+    hipLaunchKernelGGL(read_back_kernel, dim3(1), dim3(kReadBackBlock), 0, stream, (const uint8_t *)src, (uint8_t *)dst,
+                       bytes, flag, sequence);
+    return check_launch("read_back_kernel");
 }
 
 hx_status launch_copy_scan_shape(const void *src, void *dst, uint64_t bytes, hipStream_t stream) {

@@ -6,6 +6,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <memory>
 #include <mutex>
 #include <string>
@@ -75,6 +76,15 @@ struct hx_device {
     void *pinned[2] = {nullptr, nullptr};
     uint64_t pinned_bytes = 0;
     hipEvent_t pinned_ev[2] = {nullptr, nullptr};
+
+    // Pinned slots that small read-backs land in (runtime.cpp), made at
+    // hx_device_open; null where that failed.  `readback_free` has a bit per
+    // slot; a slot and its sequence belong to the thread that took the bit.
+    static constexpr uint32_t kReadBackSlots = 8;
+    static constexpr uint64_t kReadBackBytes = 4096; // data of a slot, after a 64-byte line for the flag
+    char *readback = nullptr;
+    uint64_t readback_sequence[kReadBackSlots] = {};
+    std::atomic<uint32_t> readback_free{0};
 
     // Immediate-mode buffers, one set per stream handle the caller has used
     // (created on first use, freed by hx_stream_release or at
@@ -365,6 +375,10 @@ hx_status launch_vector_op(hx_vector_op op, const float *t, const float *s, floa
 
 // Stream-ordered device-to-device copy of `bytes` bytes (a streaming kernel).
 hx_status launch_copy(const void *src, void *dst, uint64_t bytes, hipStream_t stream);
+// Stream-ordered: `bytes` of device memory to pinned host memory, then
+// `sequence` to *flag (pinned too).
+hx_status launch_read_back(const void *src, void *dst, uint32_t bytes, uint64_t *flag, uint64_t sequence,
+                           hipStream_t stream);
 // The copy in the integer scan's tile shape and order (a bench yardstick):
 // whole 128 KiB tiles, block b -> tile b.
 hx_status launch_copy_scan_shape(const void *src, void *dst, uint64_t bytes, hipStream_t stream);

@@ -5,9 +5,10 @@
 // hipMemcpy calls.
 #include "hx_internal.hpp"
 
+#include <atomic>
+#include <chrono>
 #include <cstdarg>
 #include <cstdio>
-#include <atomic>
 #include <cstring>
 #include <new>
 
@@ -296,6 +297,7 @@ hx_status hx_device_open(int32_t ordinal, hx_device **out) {
     dev->ordinal = ordinal;
     auto bail = [&](hx_status s) {
         if (dev->stream) (void)hipStreamDestroy(dev->stream);
+        if (dev->readback) (void)hipHostFree(dev->readback);
         delete dev;
         return s;
     };
@@ -361,6 +363,16 @@ hx_status hx_device_open(int32_t ordinal, hx_device **out) {
     if (err != hipSuccess)
         return bail(hip_fail(HX_ERR_DEVICE_UNAVAILABLE, err, "hipStreamCreate"));
 
+    // Pinned slots of the small read-backs; without them those take the copy engine.
+    constexpr uint64_t slots = hx_device::kReadBackSlots * (64 + hx_device::kReadBackBytes);
+    if (hipHostMalloc((void **)&dev->readback, slots, hipHostMallocMapped | hipHostMallocCoherent) == hipSuccess) {
+        std::memset(dev->readback, 0, slots);
+        dev->readback_free = (1u << hx_device::kReadBackSlots) - 1;
+    } else {
+        (void)hipGetLastError();
+        dev->readback = nullptr;
+    }
+
     // Sanity round trip (device.rs:141-163).
     void *probe = nullptr;
     err = hipMalloc(&probe, sizeof(uint32_t));
@@ -409,6 +421,7 @@ hx_status hx_device_close(hx_device *dev) {
         if (dev->pinned[i]) (void)hipHostFree(dev->pinned[i]);
         if (dev->pinned_ev[i]) (void)hipEventDestroy(dev->pinned_ev[i]);
     }
+    if (dev->readback) (void)hipHostFree(dev->readback);
     for (auto &entry : dev->immediate) {
         if (entry.second->ws) (void)hipFree(entry.second->ws);
         if (entry.second->scratch) (void)hipFree(entry.second->scratch);
@@ -572,7 +585,67 @@ hx_status staged_h2d(hx_device *dev, void *dst, const void *src, uint64_t bytes)
     return HX_OK;
 }
 
+// Waits for everything queued on the device's stream, and with bytes > 0
+// brings `bytes` of `src` to `dst`: a kernel behind the queued work writes them
+// and a flag to a pinned slot, and the host watches the flag for kWatch before
+// it blocks on the stream.  `*taken` is false, and nothing was done, when no
+// slot is free, the stream is being captured, or `src` is not the inside of
+// one allocation of this device: the caller then goes the general way.
+// us a call: 4-byte download by pageable hipMemcpyAsync and a blocking wait
+// 23.1, this way 9.6; dot product of 65536 and its download 25.7 / 13.5; copy of
+// 256 KiB and the wait 12.7 / 11.0.
+constexpr std::chrono::microseconds kWatch{200};
+hx_status read_back(hx_device *dev, void *dst, const void *src, uint64_t bytes, bool *taken) {
+    *taken = false;
+    if (!dev->readback || bytes > hx_device::kReadBackBytes) return HX_OK;
+    bool capturing = false;
+    HX_TRY(stream_capturing(dev->stream, &capturing));
+    if (capturing) return HX_OK;
+    if (bytes > 0) {
+        hipPointerAttribute_t attr;
+        hipDeviceptr_t base = nullptr;
+        size_t size = 0;
+        if (hipPointerGetAttributes(&attr, src) != hipSuccess ||
+            hipMemGetAddressRange(&base, &size, (hipDeviceptr_t)src) != hipSuccess) {
+            (void)hipGetLastError();
+            return HX_OK;
+        }
+        if (attr.type != hipMemoryTypeDevice || attr.device != dev->ordinal) return HX_OK;
+        if ((uintptr_t)src < (uintptr_t)base || (uintptr_t)src - (uintptr_t)base + bytes > size) return HX_OK;
+    }
+    uint32_t free = dev->readback_free.load(std::memory_order_relaxed);
+    while (free != 0 && !dev->readback_free.compare_exchange_weak(free, free & (free - 1), std::memory_order_acquire)) {
+    }
+    if (free == 0) return HX_OK;
+    const uint32_t slot = (uint32_t)__builtin_ctz(free);
+    char *at = dev->readback + slot * (64 + hx_device::kReadBackBytes);
+    uint64_t *flag = (uint64_t *)at;
+    const uint64_t sequence = ++dev->readback_sequence[slot];
+    auto give_back = [&] { dev->readback_free.fetch_or(1u << slot, std::memory_order_release); };
+    *taken = true;
+    const hx_status launched = launch_read_back(src, at + 64, (uint32_t)bytes, flag, sequence, dev->stream);
+    if (launched != HX_OK) {
+        give_back();
+        return launched;
+    }
+    auto arrived = [&] { return __atomic_load_n(flag, __ATOMIC_ACQUIRE) == sequence; };
+    const auto until = std::chrono::steady_clock::now() + kWatch;
+    bool seen = arrived();
+    while (!seen && std::chrono::steady_clock::now() < until) seen = arrived();
+    if (!seen) {
+        // The slot stays taken when this fails: its kernel may still write.
+        HX_HIP(hipStreamSynchronize(dev->stream), HX_ERR_TRANSFER_FAILED, "read-back synchronize");
+        if (!arrived()) return fail(HX_ERR_TRANSFER_FAILED, "the read-back kernel did not run");
+    }
+    if (bytes > 0) std::memcpy(dst, at + 64, bytes);
+    give_back();
+    return HX_OK;
+}
+
 hx_status staged_d2h(hx_device *dev, void *dst, const void *src, uint64_t bytes) {
+    bool taken = false;
+    HX_TRY(read_back(dev, dst, src, bytes, &taken));
+    if (taken) return HX_OK;
     if (bytes <= kSmallTransfer) {
         HX_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, dev->stream),
                HX_ERR_TRANSFER_FAILED, "hipMemcpyAsync D2H");
@@ -683,7 +756,9 @@ hx_status hx_copy(hx_device *dev, const void *src, uint64_t src_len, void *dst,
     HX_TRY(bind_device(dev));
     if (bytes == 0) return ok();
     HX_TRY(launch_copy(src, dst, bytes, dev->stream));
-    HX_HIP(hipStreamSynchronize(dev->stream), HX_ERR_TRANSFER_FAILED, "D2D synchronize");
+    bool taken = false;
+    HX_TRY(read_back(dev, nullptr, nullptr, 0, &taken));
+    if (!taken) HX_HIP(hipStreamSynchronize(dev->stream), HX_ERR_TRANSFER_FAILED, "D2D synchronize");
     return ok();
 }
 

@@ -1,0 +1,53 @@
+"""Small downloads: sizes around the pinned slots' and a word's, odd addresses,
+results of kernels queued just before, and more threads than slots."""
+from __future__ import annotations
+
+import threading
+
+import numpy as np
+import pytest
+
+import hephaestus_amd as hx
+from hephaestus_amd import _ffi
+
+pytestmark = pytest.mark.gpu
+
+VEC = hx.RocmDenseVectorOps()
+
+
+@pytest.mark.parametrize("skip,count", [(0, 1), (0, 4), (1, 1), (1, 7), (3, 4093), (0, 4095), (0, 4096), (2, 4096),
+                                        (0, 4097), (5, 8000)])
+def test_bytes_at_any_address(device, oracle, skip, count):
+    host = oracle.uniform_int(2048, seed=count + skip, lo=0, hi=2**32 - 1)
+    buffer = device.upload(host)
+    out = np.full(count + 2, 0xA5, np.uint8)
+    _ffi.check(_ffi.lib().hx_download(device.handle, buffer.ptr + skip, count, out.ctypes.data + 1, count, 1))
+    assert np.array_equal(out[1:-1], host.view(np.uint8)[skip:skip + count])
+    assert out[0] == 0xA5 and out[-1] == 0xA5
+
+
+def test_sees_work_queued_before(device):
+    a, b = device.upload(np.ones(1 << 20, np.float32)), device.alloc_zeroed(np.float32, 1 << 20)
+    dot = VEC.prepare_dot(device, a, a)
+    for k in range(1, 40):
+        VEC.scale_vector(device, a, 2.0 if k % 2 else 0.5)
+        assert VEC.dot_prepared(device, dot, a, a) == (4 if k % 2 else 1) * float(1 << 20)
+        VEC.copy_vector(device, a, b)
+        assert device.download_owned(b)[-1] == (2.0 if k % 2 else 1.0)
+
+
+def test_more_threads_than_slots(device):
+    buffers = [device.upload(np.arange(17, dtype=np.uint32) + 1000 * t) for t in range(20)]
+    wrong = []
+
+    def work(t):
+        for _ in range(100):
+            if not np.array_equal(device.download_owned(buffers[t]), np.arange(17, dtype=np.uint32) + 1000 * t):
+                wrong.append(t)
+
+    threads = [threading.Thread(target=work, args=(t,)) for t in range(len(buffers))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong
