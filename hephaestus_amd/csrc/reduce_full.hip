@@ -333,6 +333,13 @@ __device__ __forceinline__ typename P::Acc thread_fold(const FullParams &p, uint
     return acc;
 }
 
+// Flat operands of these sizes keep four 16-byte loads per thread in flight
+// instead of two: a thread has few trips there and the latency of each counts.
+// f32 sum, us, two / four: 2^20 4.1 / 4.2, 2^22 7.1 / 6.3, 2^24 15.0 / 14.3,
+// 30000001 22.8 / 22.0, 2^26 43.0 / 42.9, 2^27 79.1 / 80.3, 2^28 152.4 / 154.9.
+constexpr uint64_t kFourLoadsFrom = 1ull << 21;
+constexpr uint64_t kFourLoadsTo = 1ull << 26;
+
 template <typename T, int K, bool AFFINE, int MODE, int UNROLL = 2, bool NT = true>
 __global__ __launch_bounds__(kBlock) void full_reduce_kernel(FullParams p) {
     using P = Policy<T, K>;
@@ -396,7 +403,10 @@ hx_status launch_typed(const FullReduceArgs &a, void *ws, uint64_t ws_bytes, Loo
                     (unsigned long long)ws_bytes, (unsigned long long)full_reduce_workspace_bytes(a.n));
     HX_TRY(next_lookback_launch(lb, ws, ws_bytes, stream, &p.tag));
     if (a.flat) {
-        hipLaunchKernelGGL((full_reduce_kernel<T, K, AFFINE, kFlat>), dim3(blocks), dim3(kBlock), 0, stream, p);
+        if (a.n >= kFourLoadsFrom && a.n <= kFourLoadsTo)
+            hipLaunchKernelGGL((full_reduce_kernel<T, K, AFFINE, kFlat, 4>), dim3(blocks), dim3(kBlock), 0, stream, p);
+        else
+            hipLaunchKernelGGL((full_reduce_kernel<T, K, AFFINE, kFlat>), dim3(blocks), dim3(kBlock), 0, stream, p);
     } else {
         const RowsView rv = a.memory_order ? layout_rows_memory_order(a.layout) : layout_rows(a.layout);
         // The logical index a walker carries is 32 bits; argmax (the only kind
