@@ -602,7 +602,7 @@ def _colscans_u32(hx, dev, args, name, widths):
 
 
 def bench_colscan_narrow_u32(hx, dev, args):
-    """32, 64 and 128 columns: the narrow-column form (three passes)."""
+    """32, 64 and 128 columns: column strips (single pass)."""
     return _colscans_u32(hx, dev, args, "colscan_narrow_u32", (32, 64, 128))
 
 
@@ -613,7 +613,7 @@ def bench_colscan_rowtile_u32(hx, dev, args):
 
 
 def bench_colscan_rowtile_wide_u32(hx, dev, args):
-    """100 and 255 columns: three-pass row tiles."""
+    """100 and 255 columns: column strips (single pass)."""
     return _colscans_u32(hx, dev, args, "colscan_rowtile_wide_u32", (100, 255))
 
 
