@@ -162,6 +162,7 @@ SIGNATURES = {
     "hx_debug_slot16_encode": (None, [U32, U32, U64, P]),
     "hx_debug_slot16_decode": (U32, [U32, P, P]),
     "hx_debug_copy_scan_shape": (I32, [P, P, P, U64, P]),
+    "hx_debug_scan_noalloc_bytes": (I32, [I32, P, U64, LP, U32, P, U64, LP, POINTER(U64), POINTER(U64)]),
     "hx_prepare_scan": (I32, [P, I32, I32, I32, I32, P, U64, LP, U32, P, U64, LP, POINTER(P)]),
     "hx_segmented_reduce": (I32, [P, I32, I32, P, U64, P, U64, P, U64, P]),
     "hx_prepare_segmented_reduce": (I32, [P, I32, I32, P, U64, P, U64, P, U64, POINTER(P)]),

@@ -311,8 +311,8 @@ struct ScanArgs {
     uint64_t in_offset;
     int64_t out_line_stride, out_elem_stride;
     uint64_t out_offset;
-    // Column scans keep to the chunked form, whose workspace is small.
-    bool small_workspace = false;
+    // Bytes the workspace may have: strips are cut to fit (scan.hip).
+    uint64_t workspace_limit = ~0ull;
 };
 uint64_t scan_workspace_bytes(const ScanArgs &args);
 // The workspace by which hx_scan_noalloc takes or rejects a scan.
@@ -331,6 +331,8 @@ hx_status launch_scan(const ScanArgs &args, void *ws, uint64_t ws_bytes,
 hx_status lookup_noalloc_scratch(void **ptr);
 uint64_t noalloc_scratch_bytes();
 hx_status launch_scan_noalloc(const ScanArgs &args, void *scratch, hipStream_t stream);
+// The scan as launch_scan_noalloc runs it.
+ScanArgs scan_noalloc_args(const ScanArgs &args);
 
 struct SegmentedArgs {
     hx_op op;

@@ -10,7 +10,8 @@
 // the device handle; kernels and the clear kernel receive that pointer.
 //
 // The layout is that of a scan workspace: 256-byte header, then look-back
-// status words (or, for chunked column scans, chunk totals).
+// status words (or, for chunked column scans, chunk totals; strip column
+// scans whose status words would not fit take several launches).
 // The array keeps the last call's contents, so every look-back call first
 // clears the status words it will use with a fill kernel (no
 // hipMemsetAsync, which a captured graph may replay wrongly) and then runs
@@ -38,16 +39,21 @@ hx_status lookup_noalloc_scratch(void **ptr) {
     return HX_OK;
 }
 
+ScanArgs scan_noalloc_args(const ScanArgs &args) {
+    ScanArgs a = args;
+    a.workspace_limit = kNoAllocBytes;
+    return a;
+}
+
 hx_status launch_scan_noalloc(const ScanArgs &args, void *scratch_ptr, hipStream_t stream) {
     if (args.lines == 0 || args.len == 0) return HX_OK;
     const uint64_t needs = scan_fixed_workspace_bytes(args);
     if (needs > kNoAllocBytes)
         return fail(HX_ERR_DISPATCH_FAILED,
-                    "scan needs %llu bytes of workspace; the no-allocation scratch holds %llu "
+                    "scan counts for %llu bytes of workspace; the no-allocation scratch holds %llu "
                     "(use hx_scan or hx_prepare_scan)",
                     (unsigned long long)needs, (unsigned long long)kNoAllocBytes);
-    ScanArgs a = args;
-    a.small_workspace = scan_workspace_bytes(a) > kNoAllocBytes;
+    const ScanArgs a = scan_noalloc_args(args);
     const uint64_t bytes = scan_workspace_bytes(a);
     if (bytes > kNoAllocBytes)
         return fail(HX_ERR_DISPATCH_FAILED, "scan needs %llu bytes of workspace; the no-allocation scratch holds %llu",

@@ -518,6 +518,18 @@ hx_status hx_scan(hx_device *dev, hx_op op, hx_dtype dtype, hx_scan_kind kind,
 
 uint64_t hx_noalloc_scratch_bytes(void) { return noalloc_scratch_bytes(); }
 
+hx_status hx_debug_scan_noalloc_bytes(hx_dtype dtype, const void *in, uint64_t in_buf_len, const hx_layout *in_layout,
+                                      uint32_t axis, const void *out, uint64_t out_buf_len,
+                                      const hx_layout *out_layout, uint64_t *needs, uint64_t *uses) {
+    if (!needs || !uses) return fail(HX_ERR_INVALID_CONFIGURATION, "null out-pointer");
+    ScanArgs a;
+    HX_TRY(plan_scan(HX_OP_SUM, dtype, HX_SCAN_INCLUSIVE, HX_SCAN_FORWARD, in, in_buf_len, in_layout, axis,
+                     const_cast<void *>(out), out_buf_len, out_layout, &a));
+    *needs = scan_fixed_workspace_bytes(a);
+    *uses = scan_workspace_bytes(scan_noalloc_args(a));
+    return ok();
+}
+
 hx_status hx_scan_noalloc(hx_device *dev, hx_op op, hx_dtype dtype, hx_scan_kind kind,
                           hx_scan_direction direction, const void *in, uint64_t in_buf_len,
                           const hx_layout *in_layout, uint32_t axis, void *out, uint64_t out_buf_len,

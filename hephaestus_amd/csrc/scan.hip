@@ -1005,11 +1005,9 @@ void scan_short_lines_kernel(ShortParams p) {
 // (axis-0 scan of a row-major matrix).  Lines that ascend in memory in both
 // operands take the strips below (col_strip_kernel), very wide integer ones
 // and those that descend the single-pass col_lookback_kernel; this chunked
-// reduce-then-scan serves fewer than 256 descending lines, many short lines
-// (col_scan_kernel alone), and scans whose status words would not fit a
-// caller's fixed workspace (ScanArgs::small_workspace).  Lanes run across
-// lines -- a wave owns 64*V adjacent
-// lines, V = 4 giving every lane one 16-byte load per step -- and the scan
+// reduce-then-scan serves fewer than 256 descending lines and many short
+// lines (col_scan_kernel alone).  Lanes run across lines -- a wave owns 64*V
+// adjacent lines, V = 4 giving every lane one 16-byte load per step -- and the scan
 // axis is cut into chunks so that thousands of waves share the work however
 // tall the matrix is:
 //   col_totals_kernel  chunk totals of every line (one read of the input);
@@ -1877,17 +1875,20 @@ template <> struct StripPolls<float> { static constexpr int value = 2; };
 // chunk * lpad + entry.  A chunk that stays unpublished for p.spin_limit polls
 // is totalled from the input by the waiter, so progress never depends on the
 // dispatch order; the value is not published (every slot has one writer).
+// `base` is the line's total before the launch's first chunk, which is chunk
+// chunk0 of the axis (a scan of one launch: 0, and the identity).
 template <typename T, typename Op, typename Status, uint64_t ROWS, bool REV>
-__device__ void strip_lookback(const ScanParams &p, const Status &st, uint64_t c, uint64_t lpad, uint64_t line,
-                               uint64_t entry, bool live, typename ColAcc<T>::type agg,
-                               typename ColAcc<T>::type &excl) {
+__device__ void strip_lookback(const ScanParams &p, const Status &st, uint64_t c, uint64_t chunk0, uint64_t lpad,
+                               uint64_t line, uint64_t entry, bool live, typename ColAcc<T>::type base,
+                               typename ColAcc<T>::type agg, typename ColAcc<T>::type &excl) {
     using A = typename ColAcc<T>::type;
     constexpr int P = StripPolls<T>::value;
-    excl = Op::template identity<A>();
     if (c == 0) {
-        if (live) st.publish_tile(entry, p.tag, kPrefix, agg);
+        excl = base;
+        if (live) st.publish_tile(entry, p.tag, kPrefix, Op::combine(excl, agg));
         return;
     }
+    excl = Op::template identity<A>();
     if (live) st.publish_tile(c * lpad + entry, p.tag, kAggregate, agg);
     bool done = !live;
     uint64_t pos = c - 1; // next chunk to consume
@@ -1928,11 +1929,12 @@ __device__ void strip_lookback(const ScanParams &p, const Status &st, uint64_t c
         if (live) {
             const T *in = (const T *)p.in + ((int64_t)p.in_offset + (int64_t)line);
 #pragma unroll 8
-            for (uint64_t i = pos * ROWS; i < (pos + 1) * ROWS; ++i) // earlier chunks are whole
+            for (uint64_t i = (chunk0 + pos) * ROWS; i < (chunk0 + pos + 1) * ROWS; ++i) // earlier chunks are whole
                 t = Op::combine(t, (A)in[(int64_t)(REV ? p.len - 1 - i : i) * p.in_elem_stride]);
         }
         if (!done) {
             const bool missing = flag[0] == kInvalid;
+            if (pos == 0) t = Op::combine(base, t); // chunk 0 publishes its prefix
             excl = Op::combine(missing ? t : val[0], excl);
             done = (!missing && flag[0] == kPrefix) || pos == 0;
         }
@@ -1947,7 +1949,10 @@ struct StripParams {
     uint32_t deal;          // StripDeal
     uint32_t cached;        // stores go through the L2 (else non-temporal)
     uint64_t lpad;          // status entries per chunk
-    uint64_t chunks;
+    uint64_t chunks;        // of this launch
+    uint64_t chunk0;        // its first chunk's position along the axis
+    const void *totals_in;  // the lines' totals before chunk0, by entry (null: none)
+    void *totals_out;       // where the totals after the launch's last chunk go (null: nowhere)
 };
 
 template <typename T, typename Op, typename Status, int W, int STEPS, bool EXCL, bool REV>
@@ -1995,8 +2000,13 @@ void col_strip_kernel(ScanParams p, StripParams sp, Status st) {
             }
         }
         A excl;
-        strip_lookback<T, Op, Status, G::kRows, REV>(p, st, c, sp.lpad, first + l, (uint64_t)g * W + l,
-                                                     lane < (int)cnt, run, excl);
+        const uint64_t entry = (uint64_t)g * W + l;
+        const bool live = lane < (int)cnt;
+        const A base = live && sp.totals_in != nullptr ? ((const A *)sp.totals_in)[entry] : aid;
+        strip_lookback<T, Op, Status, G::kRows, REV>(p, st, c, sp.chunk0, sp.lpad, first + l, entry, live, base, run,
+                                                     excl);
+        if (live && sp.totals_out != nullptr && c + 1 == sp.chunks)
+            ((A *)sp.totals_out)[entry] = Op::combine(excl, run);
         if (lane < W) s_carry[l] = excl;
         __syncthreads(); // the carry
         return;
@@ -2010,8 +2020,8 @@ void col_strip_kernel(ScanParams p, StripParams sp, Status st) {
     const uint32_t l0 = cnt < 4 ? 0u : 4 * q + 4 <= cnt ? 4 * q : cnt - 4;
     const uint32_t nv = active ? (cnt < 4 ? cnt : 4u) : 0u;
     const uint32_t part = (uint32_t)w * G::kSub + sub;
-    const uint64_t i0 = c * G::kRows + (uint64_t)part * STEPS;
-    const bool whole = (c + 1) * G::kRows <= p.len;
+    const uint64_t i0 = (sp.chunk0 + c) * G::kRows + (uint64_t)part * STEPS;
+    const bool whole = (sp.chunk0 + c + 1) * G::kRows <= p.len;
     const T tid = Op::template identity<T>();
     T x[STEPS][4];
     {
@@ -2188,7 +2198,7 @@ bool column_wide(const ScanArgs &a) {
            (a.lines >= kWideVectorLines && a.out_elem_stride % 4 == 0);
 }
 bool column_single_pass(const ScanArgs &a) {
-    return column_mode(a) && a.lines >= kSinglePassMinLines && !a.small_workspace && !column_short_lines(a) &&
+    return column_mode(a) && a.lines >= kSinglePassMinLines && !column_short_lines(a) &&
            (column_shape(a).V == 1 || column_wide(a));
 }
 
@@ -2517,9 +2527,27 @@ constexpr uint64_t kStripDealManyInt = 8, kStripDealManyF32 = 16;
 struct StripShape {
     int W = 64, steps = 16;
     StripParams sp{};
-    uint64_t blocks = 0;
+    uint64_t chunks = 0;   // of the axis; sp.chunks a launch
+    uint64_t launches = 1;
     uint32_t lds = 0; // dynamic LDS, for the blocks per CU alone
 };
+
+uint64_t strip_entry_bytes(const ScanArgs &a) { return a.dtype == HX_DTYPE_F32 ? 16u : 8u; }
+uint64_t strip_total_bytes(const ScanArgs &a) { return a.dtype == HX_DTYPE_F32 ? 8u : 4u; }
+// Status words of a launch, and between launches two rows of line totals
+// (read by one launch, written by the next).
+uint64_t strip_bytes(const ScanArgs &a, const StripShape &s) {
+    return kLookbackOffset + s.sp.chunks * s.sp.lpad * strip_entry_bytes(a) +
+           (s.launches > 1 ? 2 * s.sp.lpad * strip_total_bytes(a) : 0);
+}
+// Blocks of a launch of `chunks` chunks.
+uint64_t strip_blocks(const StripShape &s, uint64_t chunks) {
+    switch (s.sp.deal) {
+    case kDealChunks: return ceil_div(chunks, (uint64_t)kXcds) * kXcds * s.sp.groups;
+    case kDealStrips: return chunks * ceil_div((uint64_t)s.sp.groups, (uint64_t)kXcds) * kXcds;
+    default: return chunks * s.sp.groups;
+    }
+}
 
 StripShape strip_shape(const ScanArgs &a) {
     StripShape s;
@@ -2534,8 +2562,9 @@ StripShape strip_shape(const ScanArgs &a) {
     s.sp.lpad = (uint64_t)s.sp.groups * s.W;
     auto cut = [&](int steps) {
         s.steps = steps;
-        s.sp.chunks = ceil_div(a.len, steps == 8 ? (s.W == 32 ? StripGeom<32, 8>::kRows : StripGeom<64, 8>::kRows)
-                                                 : (s.W == 32 ? StripGeom<32, 16>::kRows : StripGeom<64, 16>::kRows));
+        s.chunks = ceil_div(a.len, steps == 8 ? (s.W == 32 ? StripGeom<32, 8>::kRows : StripGeom<64, 8>::kRows)
+                                              : (s.W == 32 ? StripGeom<32, 16>::kRows : StripGeom<64, 16>::kRows));
+        s.sp.chunks = s.chunks;
     };
     cut(n <= kStripSmallElems && a.len <= kStripSmallLen ? 8 : 16);
     const bool lines128 = whole_line_rows(a) && s.sp.width % 32 == 0;
@@ -2550,30 +2579,34 @@ StripShape strip_shape(const ScanArgs &a) {
             s.sp.deal = kDealStrips;
         }
     }
-    switch (s.sp.deal) {
-    case kDealChunks: s.blocks = ceil_div(s.sp.chunks, (uint64_t)kXcds) * kXcds * s.sp.groups; break;
-    case kDealStrips: s.blocks = s.sp.chunks * ceil_div((uint64_t)s.sp.groups, (uint64_t)kXcds) * kXcds; break;
-    default: s.blocks = s.sp.chunks * s.sp.groups; break;
+    // A fixed workspace too small for the statuses: 16 rows a lane halves
+    // them, and what is still too long goes in several launches, each from
+    // the totals the one before left.  The 8 MiB scratch, us, chunked
+    // (totals, carries, rescan) / so: f32 [4194304, 64] 1417 / 403, [2097152,
+    // 128] 929 / 378, u32 [8388608, 64] 1441 / 663.
+    if (strip_bytes(a, s) > a.workspace_limit && s.steps == 8) cut(16);
+    if (strip_bytes(a, s) > a.workspace_limit) {
+        const uint64_t row = s.sp.lpad * strip_entry_bytes(a);
+        const uint64_t fixed = kLookbackOffset + 2 * s.sp.lpad * strip_total_bytes(a);
+        s.sp.chunks = a.workspace_limit > fixed ? (a.workspace_limit - fixed) / row : 0;
+        if (s.sp.chunks > kXcds) s.sp.chunks = s.sp.chunks / kXcds * kXcds;
+        s.launches = s.sp.chunks > 0 ? ceil_div(s.chunks, s.sp.chunks) : 0; // 0: no room for one chunk
     }
     return s;
 }
 
 bool strip_column_scan(const ScanArgs &a) {
-    if (a.small_workspace || !column_mode(a) || a.in_line_stride != 1 || a.out_line_stride != 1) return false;
+    if (!column_mode(a) || a.in_line_stride != 1 || a.out_line_stride != 1) return false;
     if (rowtile_column_scan(a) || column_short_lines(a)) return false;
     if (column_wide(a) || a.lines >= (1ull << 31)) return false;
-    return strip_shape(a).blocks * (kStripWaves * kWave) <= 0xFFFFFFFFull;
-}
-
-uint64_t strip_bytes(const ScanArgs &a) {
     const StripShape s = strip_shape(a);
-    return kLookbackOffset + s.sp.chunks * s.sp.lpad * (a.dtype == HX_DTYPE_F32 ? 16u : 8u);
+    return s.launches > 0 && strip_blocks(s, s.sp.chunks) * (kStripWaves * kWave) <= 0xFFFFFFFFull;
 }
 
 template <typename T, typename Op, typename Status, int W, int STEPS>
 hx_status launch_strip_dir(const ScanParams &p, const StripShape &s, const Status &st, bool excl, bool rev,
                            hipStream_t stream) {
-    const dim3 grid((uint32_t)s.blocks), block(kStripWaves * kWave);
+    const dim3 grid((uint32_t)strip_blocks(s, s.sp.chunks)), block(kStripWaves * kWave);
     if (excl && rev)
         hipLaunchKernelGGL((col_strip_kernel<T, Op, Status, W, STEPS, true, true>), grid, block, s.lds, stream, p, s.sp,
                            st);
@@ -2602,18 +2635,25 @@ hx_status launch_strip_shaped(const ScanParams &p, const StripShape &s, const St
 template <typename T, typename Op>
 hx_status launch_strip(const ScanArgs &a, ScanParams p, void *ws, uint64_t ws_bytes, LookbackState &lb,
                        hipStream_t stream) {
-    const StripShape s = strip_shape(a);
-    if (ws_bytes < strip_bytes(a))
+    StripShape s = strip_shape(a);
+    if (ws_bytes < strip_bytes(a, s))
         return fail(HX_ERR_DISPATCH_FAILED, "scan workspace of %llu bytes is too small", (unsigned long long)ws_bytes);
-    HX_TRY(next_lookback_launch(lb, ws, ws_bytes, stream, &p.tag));
     uint64_t *words = (uint64_t *)((char *)ws + kLookbackOffset);
-    hx_status r;
-    if constexpr (std::is_same<T, float>::value)
-        r = launch_strip_shaped<T, Op>(p, s, F64QuadDense{words}, a.exclusive, a.reverse, stream);
-    else
-        r = launch_strip_shaped<T, Op>(p, s, PackedStatus{words}, a.exclusive, a.reverse, stream);
-    if (r == HX_OK) commit_lookback_launch(lb);
-    return r;
+    char *totals = (char *)words + s.sp.chunks * s.sp.lpad * strip_entry_bytes(a);
+    const uint64_t row = s.sp.lpad * strip_total_bytes(a), per = s.sp.chunks;
+    for (uint64_t k = 0; k < s.launches; ++k) {
+        s.sp.chunk0 = k * per;
+        s.sp.chunks = std::min(per, s.chunks - s.sp.chunk0);
+        s.sp.totals_in = k > 0 ? totals + (k % 2) * row : nullptr;
+        s.sp.totals_out = k + 1 < s.launches ? totals + ((k + 1) % 2) * row : nullptr;
+        HX_TRY(next_lookback_launch(lb, ws, ws_bytes, stream, &p.tag));
+        if constexpr (std::is_same<T, float>::value)
+            HX_TRY((launch_strip_shaped<T, Op>(p, s, F64QuadDense{words}, a.exclusive, a.reverse, stream)));
+        else
+            HX_TRY((launch_strip_shaped<T, Op>(p, s, PackedStatus{words}, a.exclusive, a.reverse, stream)));
+        commit_lookback_launch(lb);
+    }
+    return HX_OK;
 }
 
 // 16-byte scans of lines longer than one tile whose outputs start off a
@@ -2642,7 +2682,7 @@ uint32_t scan_out_head(const ScanArgs &a) {
 uint64_t scan_bytes(const ScanArgs &a) {
     if (short_line_scan(a)) return 0;
     if (rowtile_column_scan(a)) return rowtile_lb_bytes(a);
-    if (strip_column_scan(a)) return strip_bytes(a);
+    if (strip_column_scan(a)) return strip_bytes(a, strip_shape(a));
     if (column_mode(a) && column_single_pass(a)) {
         const ColLbShape c = col_lb_shape(a);
         return kLookbackOffset + c.chunks * c.lpad * (a.dtype == HX_DTYPE_F32 ? 16u : 8u);
@@ -2655,13 +2695,13 @@ uint64_t scan_bytes(const ScanArgs &a) {
     return kLookbackOffset + status_bytes(tpl * a.lines) + status_bytes(ceil_div(tpl, kSuper) * a.lines);
 }
 
-// What a fixed workspace must hold for the scan to be taken by a caller that
-// cannot allocate (hx_scan_noalloc).  For strips the requirement is fixed by
-// the matrix alone, whatever the chunks they are cut into: one status a line
-// per 240 rows from 256 lines up; below, one word a line per tile of 32768
-// elements (32, 64 and 128 dense lines) or of whole rows up to 16384, or the
-// chunk totals of padded rows.  Strips that need more than that, near the
-// limit, run chunked instead (small_workspace).
+// The size by which a caller that cannot allocate (hx_scan_noalloc) takes or
+// rejects a scan: its workspace, except for strips, which are cut to fit any
+// workspace.  Theirs is a figure of the matrix alone, however they are cut:
+// one status a line per 240 rows from 256 lines up (16 rows a lane need no
+// more than that); below, one word a line per tile of 32768 elements (32, 64
+// and 128 dense lines) or of whole rows up to 16384, or the chunk totals of
+// padded rows.
 uint64_t fixed_workspace_bytes(const ScanArgs &a) {
     if (!strip_column_scan(a)) return scan_bytes(a);
     const uint64_t word = a.dtype == HX_DTYPE_F32 ? 8u : 4u;

@@ -400,9 +400,10 @@ hx_status hx_scan(hx_device *dev, hx_op op, hx_dtype dtype, hx_scan_kind kind,
  * harnesses that forbid hipMalloc): hx_scan with the same arguments and
  * results, whose whole workspace is a fixed 8 MiB device array per GPU
  * (hx_noalloc_scratch_bytes), so it calls no hipMalloc, hipFree or
- * allocating library routine.  A scan that needs more workspace (1-D scans
- * beyond about 2^31 elements, large single-pass column scans) is rejected
- * with HX_ERR_DISPATCH_FAILED before anything is launched.  Every call on a GPU shares that GPU's array: calls
+ * allocating library routine.  A scan that counts for more workspace (1-D
+ * scans beyond about 2^31 elements, large column scans, whose figure depends
+ * on the matrix alone) is rejected with HX_ERR_DISPATCH_FAILED before
+ * anything is launched.  Every call on a GPU shares that GPU's array: calls
  * queued on one stream run in order, calls that overlap on one GPU (other
  * streams, other threads) race. */
 hx_status hx_scan_noalloc(hx_device *dev, hx_op op, hx_dtype dtype,
@@ -642,6 +643,14 @@ uint32_t hx_debug_slot16_decode(uint32_t tag, const uint32_t *dwords, uint64_t *
  * 256 KiB tiles in XCD-contiguous order. */
 hx_status hx_debug_copy_scan_shape(hx_device *dev, const void *src, void *dst,
                                    uint64_t bytes, hx_stream stream);
+/* No counterpart in the reference.  Host-only, for tests: of the inclusive
+ * forward scan hx_scan_noalloc would run for these operands (`in` and `out`
+ * are only addresses here), *needs is the workspace size by which it is
+ * taken or rejected, *uses the bytes of the scratch it then occupies. */
+hx_status hx_debug_scan_noalloc_bytes(hx_dtype dtype, const void *in, uint64_t in_buf_len,
+                                      const hx_layout *in_layout, uint32_t axis, const void *out,
+                                      uint64_t out_buf_len, const hx_layout *out_layout,
+                                      uint64_t *needs, uint64_t *uses);
 
 #ifdef __cplusplus
 } /* extern "C" */

@@ -94,17 +94,27 @@ def test_strip_scan_under_forced_fallbacks(device, oracle, limits, dtype, rows, 
         check(device, oracle, rows, cols, dtype, seed=rows, reverse=reverse, exclusive=reverse)
 
 
-def test_noalloc_scan_whose_strips_exceed_the_scratch(device):
-    """[7400000, 64] u32: two words a line per 32768 elements, which the fixed
-    scratch holds, but more status words than it holds: the chunked form runs.
-    Row r of the input is 1 where r is a multiple of 100000, else 0."""
-    rows, cols, every = 7_400_000, 64, 100_000
+# Taken by the fixed scratch, but with more status words than it holds as
+# strips are first cut: [94200, 1279] takes longer chunks, the others several
+# launches, each from the totals of the one before.  Rows at multiples of
+# `every` hold column mod 7 + 1, all others 0.
+@pytest.mark.parametrize("rows,cols,dtype,exclusive,reverse", [
+    (94_200, 1279, np.float32, False, False), (4_000_003, 64, np.float32, False, False),
+    (3_600_001, 65, np.float32, True, True), (7_400_000, 64, np.uint32, False, False)])
+def test_noalloc_scan_whose_strips_exceed_the_scratch(device, rows, cols, dtype, exclusive, reverse):
+    every = 100_000 if rows > 1_000_000 else 3_000
     assert _ffi.lib().hx_noalloc_scratch_bytes() == 8 << 20
     lay = Layout.c_contiguous([rows, cols])
-    x, out = device.alloc_zeroed(np.uint32, rows * cols), device.alloc_zeroed(np.uint32, rows * cols)
+    x, out = device.alloc_zeroed(dtype, rows * cols), device.alloc_zeroed(dtype, rows * cols)
+    weight = (np.arange(cols) % 7 + 1).astype(dtype)
     for r in range(0, rows, every):
-        device.write_sub_buffer(x, r * cols, np.ones(cols, np.uint32))
-    SCAN.scan_axis_into_noalloc(device, hx.CumSumOp, StridedView(x, lay), 0, hx.ScanDirection.Forward,
-                                StridedView(out, lay))
+        device.write_sub_buffer(x, r * cols, weight)
+    SCAN.scan_axis_into_noalloc(device, hx.CumSumOp, StridedView(x, lay), 0,
+                                hx.ScanDirection.Reverse if reverse else hx.ScanDirection.Forward,
+                                StridedView(out, lay), hx.ScanKind.Exclusive if exclusive else hx.ScanKind.Inclusive)
+    marks = np.zeros(rows, np.int64)
+    marks[::every] = 1
+    count = _numpy_scan(marks[:, None], False, exclusive, reverse)[:, 0].astype(dtype)
     got = device.download_owned(out).reshape(rows, cols)
-    assert np.array_equal(got, np.broadcast_to((np.arange(rows, dtype=np.uint32) // every + 1)[:, None], got.shape))
+    for c in range(cols):
+        assert np.array_equal(got[:, c], count * weight[c]), c
