@@ -313,14 +313,17 @@ struct ScanArgs {
     uint64_t out_offset;
     // Bytes the workspace may have: strips are cut to fit (scan.hip).
     uint64_t workspace_limit = ~0ull;
+    // The status words are cleared by a launch in front of the scan (stream
+    // capture, hx_scan_noalloc).
+    bool clears = false;
 };
 uint64_t scan_workspace_bytes(const ScanArgs &args);
 // The workspace by which hx_scan_noalloc takes or rejects a scan.
 uint64_t scan_fixed_workspace_bytes(const ScanArgs &args);
 // False for chunked column scans, whose workspace holds chunk totals
 // instead of look-back status words (immediate calls take it from device
-// scratch), and for short dense lines, which need none; true for every other
-// scan.
+// scratch), and for scans that need none (short dense lines, column scans of
+// one tile or chunk); true for every other scan.
 bool scan_uses_lookback(const ScanArgs &args);
 hx_status launch_scan(const ScanArgs &args, void *ws, uint64_t ws_bytes,
                       LookbackState &st, hipStream_t stream);
@@ -414,6 +417,7 @@ struct hx_plan {
     std::mutex mu;
     virtual ~hx_plan();
     virtual hx_status dispatch(hipStream_t stream) = 0;
-    // Whether dispatch() draws a look-back tag for words in ws.
+    // Whether a captured dispatch() uses tagged words in ws (lookback.captured
+    // is set when it is asked, and for the dispatch).
     virtual bool tagged() const { return false; }
 };

@@ -42,6 +42,7 @@ hx_status lookup_noalloc_scratch(void **ptr) {
 ScanArgs scan_noalloc_args(const ScanArgs &args) {
     ScanArgs a = args;
     a.workspace_limit = kNoAllocBytes;
+    a.clears = true;
     return a;
 }
 

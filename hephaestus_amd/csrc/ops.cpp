@@ -289,9 +289,19 @@ hx_status plan_scan(hx_op op, hx_dtype dtype, hx_scan_kind kind, hx_scan_directi
 
 struct ScanPlan final : hx_plan {
     ScanArgs args;
-    bool tagged() const override { return scan_uses_lookback(args); }
+    // Under capture some scans take a form without status words, which
+    // needs no more workspace than the plan's.
+    ScanArgs launch_args() const {
+        ScanArgs a = args;
+        a.clears = lookback.captured;
+        return a;
+    }
+    bool tagged() const override {
+        const ScanArgs a = launch_args();
+        return scan_uses_lookback(a) && scan_workspace_bytes(a) > kLookbackOffset;
+    }
     hx_status dispatch(hipStream_t stream) override {
-        return launch_scan(args, ws, ws_bytes, lookback, stream);
+        return launch_scan(launch_args(), ws, ws_bytes, lookback, stream);
     }
 };
 

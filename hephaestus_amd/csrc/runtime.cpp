@@ -825,11 +825,12 @@ namespace {
 hx_status dispatch_locked(hx_plan *plan, hipStream_t s) {
     bool capturing = false;
     HX_TRY(stream_capturing(s, &capturing));
-    if (!capturing || !plan->tagged()) return plan->dispatch(s);
-    if (plan->ws_bytes > kLookbackOffset)
-        HX_TRY(launch_clear_words((char *)plan->ws + kLookbackOffset, (plan->ws_bytes - kLookbackOffset) / 8, s));
+    if (!capturing) return plan->dispatch(s);
     plan->lookback.captured = true;
-    const hx_status st = plan->dispatch(s);
+    hx_status st = HX_OK;
+    if (plan->tagged() && plan->ws_bytes > kLookbackOffset)
+        st = launch_clear_words((char *)plan->ws + kLookbackOffset, (plan->ws_bytes - kLookbackOffset) / 8, s);
+    if (st == HX_OK) st = plan->dispatch(s);
     plan->lookback.captured = false;
     return st;
 }

@@ -1365,7 +1365,8 @@ __device__ __forceinline__ void row_group_rescan(T *tile, uint32_t n, uint32_t C
 // folded in group order, so integers match the owner's bits and f32 its value
 // to rounding) and uses it, so progress never depends on dispatch order.  The round's needed values fold over k through an LDS tree
 // into the column carry, which is published with the tile's aggregate as the
-// inclusive prefix.  Tile 0's value is always its prefix.  f32 carries are
+// inclusive prefix.  Tile 0's value is always its prefix; an only tile
+// publishes nothing.  f32 carries are
 // f64 in 16-byte slots (F64QuadDense), integers packed words.  An f32
 // carry's f64 rounding depends on which predecessors had published prefixes:
 // results agree with the f64 scan to within its bound, not bit for bit across
@@ -1421,7 +1422,7 @@ void col_rowtile_lookback_kernel(ScanParams p, RowTileShape s, Status st) {
     if (j < C) {
         const A tot = gtot[(s.groups - 1) * C + j];
         s_agg[j] = tot;
-        st.publish_tile(t * C + j, p.tag, t == 0 ? kPrefix : kAggregate, tot);
+        if (s.tiles > 1) st.publish_tile(t * C + j, p.tag, t == 0 ? kPrefix : kAggregate, tot);
         s_carry[j] = aid;
         s_done[j] = t == 0 ? 1u : 0u;
     }
@@ -1877,15 +1878,17 @@ template <> struct StripPolls<float> { static constexpr int value = 2; };
 // dispatch order; the value is not published (every slot has one writer).
 // `base` is the line's total before the launch's first chunk, which is chunk
 // chunk0 of the axis (a scan of one launch: 0, and the identity).
+// A launch of one chunk publishes nothing (its status area is not allocated).
 template <typename T, typename Op, typename Status, uint64_t ROWS, bool REV>
-__device__ void strip_lookback(const ScanParams &p, const Status &st, uint64_t c, uint64_t chunk0, uint64_t lpad,
-                               uint64_t line, uint64_t entry, bool live, typename ColAcc<T>::type base,
-                               typename ColAcc<T>::type agg, typename ColAcc<T>::type &excl) {
+__device__ void strip_lookback(const ScanParams &p, const Status &st, uint64_t c, uint64_t chunks, uint64_t chunk0,
+                               uint64_t lpad, uint64_t line, uint64_t entry, bool live,
+                               typename ColAcc<T>::type base, typename ColAcc<T>::type agg,
+                               typename ColAcc<T>::type &excl) {
     using A = typename ColAcc<T>::type;
     constexpr int P = StripPolls<T>::value;
     if (c == 0) {
         excl = base;
-        if (live) st.publish_tile(entry, p.tag, kPrefix, Op::combine(excl, agg));
+        if (live && chunks > 1) st.publish_tile(entry, p.tag, kPrefix, Op::combine(excl, agg));
         return;
     }
     excl = Op::template identity<A>();
@@ -2003,8 +2006,8 @@ void col_strip_kernel(ScanParams p, StripParams sp, Status st) {
         const uint64_t entry = (uint64_t)g * W + l;
         const bool live = lane < (int)cnt;
         const A base = live && sp.totals_in != nullptr ? ((const A *)sp.totals_in)[entry] : aid;
-        strip_lookback<T, Op, Status, G::kRows, REV>(p, st, c, sp.chunk0, sp.lpad, first + l, entry, live, base, run,
-                                                     excl);
+        strip_lookback<T, Op, Status, G::kRows, REV>(p, st, c, sp.chunks, sp.chunk0, sp.lpad, first + l, entry,
+                                                     live, base, run, excl);
         if (live && sp.totals_out != nullptr && c + 1 == sp.chunks)
             ((A *)sp.totals_out)[entry] = Op::combine(excl, run);
         if (lane < W) s_carry[l] = excl;
@@ -2302,16 +2305,16 @@ constexpr int kLongWaves = 8, kLongSteps = 16;
 // 10^5 elements 7.4 (8.4) -> 4.0 (4.1), 10^6 7.2 (7.9) -> 5.1 (5.9), 3 * 10^6
 // 9.1 (9.5) -> 6.4 (7.2), 10^7 15.4 (14.9) -> 14.5 (13.8); 16 * 10^6 in 8192s 26.8
 // against 20.4.
+// Chained tiles have status words.  Where a launch of its own clears them
+// (ScanArgs::clears) a line that one tile holds keeps it up to kClearOneTile
+// elements, and beyond where it fills the tile: a graph node of u32 lines of
+// 2049 / 8192 / 32768 elements 3.1 / 3.1 / 5.1 us against 5.3 / 5.1 / 5.3 for clear
+// and scan, but 12000 6.2 against 5.2 (a tile that is not full loads element
+// by element).
 constexpr uint64_t kMidMaxLines = 255;
 constexpr uint64_t kMid2048Elems = 1ull << 17, kMid4096Elems = 1ull << 22, kMid8192Elems = 10ull << 20;
-inline TileShape tile_shape(const ScanArgs &a) {
-    const uint64_t len = a.len, n = a.len * a.lines;
-    if (len > 2048 && a.lines <= kMidMaxLines && a.in_elem_stride == 1 && a.out_elem_stride == 1) {
-        const bool grid = ((uintptr_t)a.out + 4u * a.out_offset + (a.reverse ? 4u * len : 0u)) % 128 == 0;
-        if (n <= kMid2048Elems) return {2, 4};
-        if (n <= kMid4096Elems) return {4, 4};
-        if (len > 4096 && n <= (grid ? kMid8192Elems : 1ull << 23)) return {4, 8};
-    }
+constexpr uint64_t kClearOneTile = 8192;
+inline TileShape line_tile_shape(uint64_t len) {
     if (len <= 256) return {1, 1};
     if (len <= 512) return {1, 2};
     if (len <= 1024) return {2, 2};
@@ -2321,6 +2324,18 @@ inline TileShape tile_shape(const ScanArgs &a) {
     if (len <= 16384) return {4, 16};
     if (len <= 32768) return {kWaves, kSteps};
     return TileShape{kLongWaves, kLongSteps};
+}
+inline TileShape tile_shape(const ScanArgs &a) {
+    const uint64_t len = a.len, n = a.len * a.lines;
+    const TileShape one = line_tile_shape(len);
+    const bool keep_one = a.clears && len <= one.elems() && (len <= kClearOneTile || len == one.elems());
+    if (len > 2048 && !keep_one && a.lines <= kMidMaxLines && a.in_elem_stride == 1 && a.out_elem_stride == 1) {
+        const bool grid = ((uintptr_t)a.out + 4u * a.out_offset + (a.reverse ? 4u * len : 0u)) % 128 == 0;
+        if (n <= kMid2048Elems) return {2, 4};
+        if (n <= kMid4096Elems) return {4, 4};
+        if (len > 4096 && n <= (grid ? kMid8192Elems : 1ull << 23)) return {4, 8};
+    }
+    return one;
 }
 bool long_tiles(const TileShape &s) { return s.waves == kLongWaves && s.steps == kLongSteps; }
 
@@ -2452,6 +2467,7 @@ bool rowtile_column_scan(const ScanArgs &a) {
 
 uint64_t rowtile_lb_bytes(const ScanArgs &a) {
     const RowTileShape s = row_tile_shape(a.lines, a.len);
+    if (s.tiles <= 1) return 0; // no look-back, no status words
     return kLookbackOffset + s.tiles * a.lines * (a.dtype == HX_DTYPE_F32 ? 16u : 8u);
 }
 
@@ -2473,7 +2489,7 @@ hx_status launch_rowtile_lb(const ScanArgs &a, ScanParams p, void *ws, uint64_t 
     if (s.tiles > 0x7FFFFFFFull) return fail(HX_ERR_DISPATCH_FAILED, "column scan exceeds the grid range");
     if (ws_bytes < rowtile_lb_bytes(a))
         return fail(HX_ERR_DISPATCH_FAILED, "scan workspace of %llu bytes is too small", (unsigned long long)ws_bytes);
-    HX_TRY(next_lookback_launch(lb, ws, ws_bytes, stream, &p.tag));
+    if (s.tiles > 1) HX_TRY(next_lookback_launch(lb, ws, ws_bytes, stream, &p.tag));
     p.tile0 = 0;
     uint64_t *words = (uint64_t *)((char *)ws + kLookbackOffset);
     hx_status r;
@@ -2486,7 +2502,7 @@ hx_status launch_rowtile_lb(const ScanArgs &a, ScanParams p, void *ws, uint64_t 
         r = a.exclusive ? launch_rowtile_lb_dir<T, Op, PackedStatus, true>(p, s, st, a.reverse, stream)
                         : launch_rowtile_lb_dir<T, Op, PackedStatus, false>(p, s, st, a.reverse, stream);
     }
-    if (r == HX_OK) commit_lookback_launch(lb);
+    if (r == HX_OK && s.tiles > 1) commit_lookback_launch(lb);
     return r;
 }
 
@@ -2535,8 +2551,9 @@ struct StripShape {
 uint64_t strip_entry_bytes(const ScanArgs &a) { return a.dtype == HX_DTYPE_F32 ? 16u : 8u; }
 uint64_t strip_total_bytes(const ScanArgs &a) { return a.dtype == HX_DTYPE_F32 ? 8u : 4u; }
 // Status words of a launch, and between launches two rows of line totals
-// (read by one launch, written by the next).
+// (read by one launch, written by the next); nothing for one chunk.
 uint64_t strip_bytes(const ScanArgs &a, const StripShape &s) {
+    if (s.chunks <= 1) return 0;
     return kLookbackOffset + s.sp.chunks * s.sp.lpad * strip_entry_bytes(a) +
            (s.launches > 1 ? 2 * s.sp.lpad * strip_total_bytes(a) : 0);
 }
@@ -2646,12 +2663,12 @@ hx_status launch_strip(const ScanArgs &a, ScanParams p, void *ws, uint64_t ws_by
         s.sp.chunks = std::min(per, s.chunks - s.sp.chunk0);
         s.sp.totals_in = k > 0 ? totals + (k % 2) * row : nullptr;
         s.sp.totals_out = k + 1 < s.launches ? totals + ((k + 1) % 2) * row : nullptr;
-        HX_TRY(next_lookback_launch(lb, ws, ws_bytes, stream, &p.tag));
+        if (s.chunks > 1) HX_TRY(next_lookback_launch(lb, ws, ws_bytes, stream, &p.tag));
         if constexpr (std::is_same<T, float>::value)
             HX_TRY((launch_strip_shaped<T, Op>(p, s, F64QuadDense{words}, a.exclusive, a.reverse, stream)));
         else
             HX_TRY((launch_strip_shaped<T, Op>(p, s, PackedStatus{words}, a.exclusive, a.reverse, stream)));
-        commit_lookback_launch(lb);
+        if (s.chunks > 1) commit_lookback_launch(lb);
     }
     return HX_OK;
 }
@@ -2804,7 +2821,7 @@ uint64_t scan_fixed_workspace_bytes(const ScanArgs &a) { return fixed_workspace_
 
 bool scan_uses_lookback(const ScanArgs &a) {
     if (short_line_scan(a)) return false;
-    if (rowtile_column_scan(a) || strip_column_scan(a)) return true;
+    if (rowtile_column_scan(a) || strip_column_scan(a)) return scan_bytes(a) > 0; // one tile or chunk: none
     return !column_mode(a) || column_single_pass(a);
 }
 
