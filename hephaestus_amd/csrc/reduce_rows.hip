@@ -831,7 +831,9 @@ constexpr uint64_t kTargetWaves = 2048;
 // Lines per column-tile chunk, at least; half as many up to kShortCols lines,
 // where 32 leave CUs without a wave (f32 sum, us, 32 -> 16 lines a chunk:
 // 1779 x 1398 9.0 -> 7.7, 3000 x 837 8.6 -> 7.6, 5000 x 506 9.0 -> 7.8;
-// 10000 x 506 9.7 -> 10.7, 30000 x 195 11.0 -> 13.4).
+// 10000 x 506 9.7 -> 10.7, 30000 x 195 11.0 -> 13.4).  Up to kMinColChunk lines
+// stay whole: two chunks and a fold take 17 x 2049 from 3.3 to 5.3, 18 x 205844
+// from 3.5 to 12.7 and 32 x 100001 from 3.7 to 8.8.
 constexpr uint64_t kMinColChunk = 32;
 constexpr uint64_t kShortCols = 4096;
 constexpr uint64_t kMinRowChunk = 8192;  // elements per split-row chunk
@@ -977,9 +979,13 @@ Shape plan_shape(const RowParams &p, bool cols_layout) {
         }
         if (s.groups < kTargetWaves) {
             // No more than kTargetWaves: a few beyond leave some CUs a block
-            // more than the others (20000 x 12000 f32 sum 180 -> 153 us.  Above half of it two chunks all the same.
+            // more than the others (20000 x 12000 f32 sum 180 -> 153 us).
+            // Above half of kTargetWaves groups, two chunks all the same.
             k = s.groups <= kTargetWaves / 2 ? kTargetWaves / s.groups : 2;
-            const uint64_t kmax = ceil_div(p.cols, p.cols <= kShortCols ? kMinColChunk / 2 : kMinColChunk);
+            const uint64_t kmin = p.cols <= kMinColChunk ? p.cols
+                                  : p.cols <= kShortCols ? kMinColChunk / 2
+                                                         : kMinColChunk;
+            const uint64_t kmax = ceil_div(p.cols, kmin);
             if (k > kmax) k = kmax;
         }
     } else {
