@@ -509,7 +509,11 @@ template <int V> __device__ __forceinline__ uint64_t cols_first_output(uint64_t 
 // Statistics of lines [j0, j1) of the 64*V adjacent outputs from o0 (V per
 // lane) of a column tile, kU lines in flight per lane: V = 4 gives every
 // lane one 16-byte load per line, so each load instruction of a wave covers
-// 1 KiB of one line.
+// 1 KiB of one line.  The last lines go in batches of 4 (2 and 1): one by one
+// they are a memory round trip each, and a whole batch with the last line
+// loaded again in place of the missing ones costs its bandwidth.  f32 sum, us,
+// repeated lines / so: 2 x 16000001 65 / 39, 4 x 16000001 73 / 56, 320 x 30003 9.3
+// / 7.3, 64 x 10001 4.1 / 3.6, 200 x 301 3.8 / 3.5.
 template <typename T, bool AFFINE, int FLAGS, int V>
 __device__ __forceinline__ void cols_walk(const RowParams &p, uint64_t o0, uint64_t j0, uint64_t j1,
                                           Stats<T, FLAGS> (&st)[V]) {
@@ -524,38 +528,33 @@ __device__ __forceinline__ void cols_walk(const RowParams &p, uint64_t o0, uint6
             st[2].visit(prologue<T, AFFINE>((T)x.z, p.a, p.b), jj);
             st[3].visit(prologue<T, AFFINE>((T)x.w, p.a, p.b), jj);
         };
-        for (; j + kU <= j1; j += kU) {
-            Vt x[kU];
+        auto batch = [&](auto count) {
+            constexpr int N = decltype(count)::value;
+            Vt x[N];
 #pragma unroll
-            for (int u = 0; u < kU; ++u)
+            for (int u = 0; u < N; ++u)
                 x[u] = __builtin_nontemporal_load((const Vt *)(base + (int64_t)(j + u) * p.col_stride));
 #pragma unroll
-            for (int u = 0; u < kU; ++u) visit(x[u], (uint32_t)(j + u));
-        }
-        // The last lines together as well (past the end: the last one again,
-        // not visited): taken one by one they are a memory round trip each.
-        if (j < j1) {
-            Vt x[kU];
-#pragma unroll
-            for (int u = 0; u < kU; ++u) {
-                const uint64_t l = j + u < j1 ? j + u : j1 - 1;
-                x[u] = __builtin_nontemporal_load((const Vt *)(base + (int64_t)l * p.col_stride));
-            }
-#pragma unroll
-            for (int u = 0; u < kU; ++u)
-                if (j + u < j1) visit(x[u], (uint32_t)(j + u));
-        }
+            for (int u = 0; u < N; ++u) visit(x[u], (uint32_t)(j + u));
+            j += N;
+        };
+        while (j + kU <= j1) batch(std::integral_constant<int, kU>{});
+        if (j + 4 <= j1) batch(std::integral_constant<int, 4>{});
+        if (j + 2 <= j1) batch(std::integral_constant<int, 2>{});
+        if (j < j1) batch(std::integral_constant<int, 1>{});
     } else {
-        for (; j + kU <= j1; j += kU) {
-            T x[kU];
+        auto batch = [&](auto count) {
+            constexpr int N = decltype(count)::value;
+            T x[N];
 #pragma unroll
-            for (int u = 0; u < kU; ++u) x[u] = __builtin_nontemporal_load(base + (int64_t)(j + u) * p.col_stride);
+            for (int u = 0; u < N; ++u) x[u] = __builtin_nontemporal_load(base + (int64_t)(j + u) * p.col_stride);
 #pragma unroll
-            for (int u = 0; u < kU; ++u) st[0].visit(prologue<T, AFFINE>(x[u], p.a, p.b), (uint32_t)(j + u));
-        }
-        for (; j < j1; ++j)
-            st[0].visit(prologue<T, AFFINE>(__builtin_nontemporal_load(base + (int64_t)j * p.col_stride), p.a, p.b),
-                        (uint32_t)j);
+            for (int u = 0; u < N; ++u) st[0].visit(prologue<T, AFFINE>(x[u], p.a, p.b), (uint32_t)(j + u));
+            j += N;
+        };
+        while (j + kU <= j1) batch(std::integral_constant<int, kU>{});
+        while (j + 4 <= j1) batch(std::integral_constant<int, 4>{});
+        while (j < j1) batch(std::integral_constant<int, 1>{});
     }
 }
 
