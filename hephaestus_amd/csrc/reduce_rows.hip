@@ -499,9 +499,7 @@ __global__ __launch_bounds__(kBlock) void rows_tile_kernel(RowParams p, uint32_t
 
 // First of the V outputs of the lane that `want` falls to.  Where the outputs
 // are no multiple of 4 the last lane moves back to a whole vector: it shares
-// outputs with its neighbour, and both write the same bits.  With one output
-// per lane such matrices took, f32 sum with its fold: [23542, 573] 18.9 us
-// against 16.6, [10000, 4099] 42.6 against 33, [56667, 1830] 93 against 72.
+// outputs with its neighbour, and both write the same bits.
 template <int V> __device__ __forceinline__ uint64_t cols_first_output(uint64_t want, uint64_t outputs) {
     return V == 4 && want + 4 > outputs ? outputs - 4 : want;
 }
@@ -853,7 +851,7 @@ constexpr uint64_t kRowTargetWaves = 4096; // split rows when fewer than half th
 // 1500 x 256 5.8 / 8.0, 2048 x 256 6.4 / 7.6, 2048 x 100 12.7 / 7.8,
 // 2500 x 8192 20 / 19, 2500 x 12000 20 / 26, 5000 x 12000 38 / 44,
 // 5000 x 30000 100 / 97.
-// Strided outputs: a lane per output and a serial slice per wave, up to
+// One output a lane (column_vectors): a serial slice per wave, up to
 // kBlockFoldLines lines and kBlockFoldElems elements.
 constexpr uint64_t kBlockFoldLines = 64 * kFoldSlices;
 constexpr uint64_t kBlockFoldElems = 1ull << 20;
@@ -891,6 +889,38 @@ struct Shape {
     uint64_t groups = 0, chunk = 0;
     uint32_t nchunks = 1;
 };
+
+// Whether the lanes of a column reduction take 16-byte vectors of four
+// outputs (at 4-byte alignment, Vec4A4: any line start) or one output each.
+// Output counts that are multiples of 4 always take vectors.  The others
+// measured, f32 sum, us, one output / vectors:
+//   up to 32 lines, a lane each: 17 x 2049 2.7 / 3.2, 32 x 10241 2.9 / 3.5, 24 x
+//     200001 3.8 / 4.9, but 24 x 500001 9.2 / 7.8: vectors from kVectorWide
+//     outputs.
+//   blocks up to kBlockFoldElems elements: the merges of four outputs cost
+//     more than wider loads gain, 33 x 2049 2.8 / 3.5, 256 x 301 3.3 / 3.8, until
+//     a last group of a few outputs fetches its lines almost alone, 700 x 65
+//     5.5 / 4.4, 1024 x 257 6.2 / 4.7.
+//   beyond that many elements, up to kBlockFoldLines lines: 256 x 10241 6.6 / 3.8.
+//   more lines: a wave of vectors has few lanes at few outputs, 10^6 x 11
+//     (padded) 22 / 78, 6000 x 201 6.0 / 6.8, 100000 x 193 17.5 / 21.5.  Vectors
+//     from kVectorElems elements, 300000 x 259 63.6 / 55.4, and at more outputs
+//     with many lines, 6000 x 1001 9.7 / 8.8, 4096 x 1001 6.9 / 7.9.
+constexpr uint64_t kVectorWide = 1ull << 18;
+constexpr uint64_t kVectorMinCols = 640, kVectorMinLines = 5000, kVectorElems = 3ull << 23;
+constexpr uint64_t kLastGroup = 8, kLastGroupLines = 256;
+bool column_vectors(const RowParams &p, uintptr_t base) {
+    if (p.row_stride != 1 || p.rows < 4 || base % 4 != 0) return false;
+    if (p.rows % 4 == 0) return true;
+    const uint64_t lines = p.cols, outputs = p.rows;
+    if (lines <= kMinColChunk) return outputs >= kVectorWide;
+    if (lines <= kBlockFoldLines) {
+        const uint64_t last = outputs % kWave;
+        return outputs * lines > kBlockFoldElems || (lines > kLastGroupLines && last > 0 && last <= kLastGroup);
+    }
+    return outputs >= kBlockManyCols || (outputs >= kVectorMinCols && lines >= kVectorMinLines) ||
+           (outputs >= 2 * kWave && outputs * lines >= kVectorElems);
+}
 
 // Whether a column reduction takes cols_block_kernel, and its lanes and waves
 // (s.vec and s.groups, the groups of 64 lanes, are set).
@@ -966,8 +996,7 @@ Shape plan_shape(const RowParams &p, bool cols_layout) {
         return s;
     }
     if (cols_layout) {
-        // 16-byte vectors at 4-byte alignment (Vec4A4): any line start.
-        s.vec = p.row_stride == 1 && p.rows >= 4 && base % 4 == 0;
+        s.vec = column_vectors(p, base);
         s.V = s.vec ? 4 : 1;
         s.groups = ceil_div(p.rows, (uint64_t)kWave * s.V);
         if (block_columns(p, s)) {
