@@ -924,6 +924,12 @@ bool column_vectors(const RowParams &p, uintptr_t base) {
 
 // Whether a column reduction takes cols_block_kernel, and its lanes and waves
 // (s.vec and s.groups, the groups of 64 lanes, are set).
+// Launches of 2^32 and more work-items (reachable where lines overlap in
+// memory) are left to the column tiles, whose waves each take more outputs.
+bool block_fits(const RowParams &p, const Shape &s) {
+    const uint64_t blocks = ceil_div(ceil_div(p.rows, (uint64_t)s.lanes * s.V), 8) * 8;
+    return blocks * (uint64_t)(kWave * s.block_waves) <= 0xFFFFFFFFull;
+}
 bool block_columns(const RowParams &p, Shape &s) {
     if (p.cols <= kMinColChunk) return false;
     if (!s.vec)
@@ -932,11 +938,11 @@ bool block_columns(const RowParams &p, Shape &s) {
         const uint64_t rounds = ceil_div(s.groups, kCus);
         const bool even = rounds == 1 || rounds * kCus * 4 <= s.groups * 5;
         s.block_waves = kWideWaves;
-        if (p.cols <= 512 || (p.cols <= kWideLines && even)) return true;
+        if (p.cols <= 512 || (p.cols <= kWideLines && even)) return block_fits(p, s);
     }
     s.lanes = kBlockLanes;
     s.block_waves = kFoldSlices;
-    return p.cols <= (p.rows >= kBlockManyCols ? 4 : 1) * kBlockFoldLines;
+    return p.cols <= (p.rows >= kBlockManyCols ? 4 : 1) * kBlockFoldLines && block_fits(p, s);
 }
 
 // Lanes per row: the largest group that still gives each lane at least
