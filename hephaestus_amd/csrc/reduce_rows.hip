@@ -1016,10 +1016,9 @@ Shape plan_shape(const RowParams &p, bool cols_layout) {
             // more than the others (20000 x 12000 f32 sum 180 -> 153 us).
             // Above half of kTargetWaves groups, two chunks all the same.
             k = s.groups <= kTargetWaves / 2 ? kTargetWaves / s.groups : 2;
-            const uint64_t kmin = p.cols <= kMinColChunk ? p.cols
-                                  : p.cols <= kShortCols ? kMinColChunk / 2
-                                                         : kMinColChunk;
-            const uint64_t kmax = ceil_div(p.cols, kmin);
+            const uint64_t kmax = p.cols <= kMinColChunk
+                                      ? 1 // none for an empty axis
+                                      : ceil_div(p.cols, p.cols <= kShortCols ? kMinColChunk / 2 : kMinColChunk);
             if (k > kmax) k = kmax;
         }
     } else {

@@ -22,3 +22,14 @@ def test_few_lines_are_one_launch(device, oracle, lines, cols, pitch):
         StridedView(out, Layout.c_contiguous([1, cols])))
     assert plan.workspace_bytes() == 0
     blocks.test_column_reductions(device, oracle, lines, cols, pitch, 0)
+
+
+@pytest.mark.parametrize("cols", [1, 3, 64, 1001])
+def test_no_lines(device, cols):
+    """An empty reduced axis: the identity, one launch."""
+    x, out = device.alloc_zeroed(np.uint32, 0), device.upload(np.full(cols, 7, np.uint32))
+    ops = hx.RocmAxisReductionOps()
+    views = StridedView(x, Layout.c_contiguous([0, cols])), StridedView(out, Layout.c_contiguous([1, cols]))
+    assert ops.prepare_reduce_axis_into(device, hx.SumOp, views[0], 0, views[1]).workspace_bytes() == 0
+    ops.reduce_axis_into(device, hx.SumOp, views[0], 0, views[1])
+    assert not device.download_owned(out).any()
