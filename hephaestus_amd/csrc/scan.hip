@@ -1134,34 +1134,51 @@ __global__ __launch_bounds__(kBlock) void col_totals_kernel(ScanParams p, typena
         if ((uint32_t)v < nv) totals[w.k * p.lines + w.line0 + v] = acc[v];
 }
 
-// Exclusive scan of each line's chunk totals, in place.  A block owns 64
-// lines (lanes) and kCarrySlices waves; wave s totals its contiguous range of
-// chunks, the slice totals are scanned through LDS, and each wave rewrites
-// its range from its slice carry.
-constexpr int kCarrySlices = 16;
+// Exclusive scan of each line's chunk totals, in place.  A block owns 16 lines
+// and cuts the chunks into 64 contiguous slices, one to every 16 lanes: a lane
+// totals its slice, kCarryBatch loads together (one batch, kept for the
+// rewrite, up to 512 chunks), folds the earlier slices' totals through LDS and
+// rewrites its slice.  The order depends on the chunk count alone.  With
+// slices of a sixteenth of the chunks and one load at a time, [65536, 100] f32
+// in three launches took 33.4 us against 25.4.
+constexpr int kCarryWaves = 16, kCarryLines = 16, kCarryBatch = 8;
+constexpr int kCarrySlices = kCarryWaves * (kWave / kCarryLines);
 
 template <typename A, typename Op>
-__global__ __launch_bounds__(kWave *kCarrySlices) void col_carry_kernel(A *totals, uint64_t lines,
-                                                                        uint32_t nchunks) {
-    __shared__ A sh[kCarrySlices * kWave];
-    const int lane = lane_id();
-    const int s = threadIdx.x / kWave;
-    const uint64_t line = (uint64_t)blockIdx.x * kWave + lane;
+__global__ __launch_bounds__(kWave *kCarryWaves) void col_carry_kernel(A *totals, uint64_t lines, uint32_t nchunks) {
+    __shared__ A sh[kCarrySlices][kCarryLines];
+    const int q = threadIdx.x % kCarryLines;
+    const uint32_t s = threadIdx.x / kCarryLines;
+    const uint64_t line = (uint64_t)blockIdx.x * kCarryLines + q;
     const uint32_t per = (nchunks + kCarrySlices - 1) / kCarrySlices;
     const uint32_t k0 = s * per < nchunks ? s * per : nchunks;
     const uint32_t k1 = k0 + per < nchunks ? k0 + per : nchunks;
-    A t = Op::template identity<A>();
-    if (line < lines)
-        for (uint32_t k = k0; k < k1; ++k) t = Op::combine(t, totals[(uint64_t)k * lines + line]);
-    sh[s * kWave + lane] = t;
+    const bool live = line < lines;
+    const A id = Op::template identity<A>();
+    A v[kCarryBatch];
+    auto load = [&](uint32_t k) {
+#pragma unroll
+        for (uint32_t u = 0; u < kCarryBatch; ++u)
+            v[u] = live && k + u < k1 ? totals[(uint64_t)(k + u) * lines + line] : id;
+    };
+    A sum = id;
+    for (uint32_t k = k0; k < k1; k += kCarryBatch) {
+        load(k);
+#pragma unroll
+        for (uint32_t u = 0; u < kCarryBatch; ++u) sum = Op::combine(sum, v[u]);
+    }
+    sh[s][q] = sum;
     __syncthreads();
-    if (line >= lines) return;
-    A acc = Op::template identity<A>();
-    for (int q = 0; q < s; ++q) acc = Op::combine(acc, sh[q * kWave + lane]);
-    for (uint32_t k = k0; k < k1; ++k) {
-        const A v = totals[(uint64_t)k * lines + line];
-        totals[(uint64_t)k * lines + line] = acc;
-        acc = Op::combine(acc, v);
+    A acc = id;
+#pragma unroll 8
+    for (uint32_t t = 0; t < s; ++t) acc = Op::combine(acc, sh[t][q]);
+    for (uint32_t k = k0; k < k1; k += kCarryBatch) {
+        if (per > (uint32_t)kCarryBatch) load(k);
+#pragma unroll
+        for (uint32_t u = 0; u < kCarryBatch; ++u) {
+            if (live && k + u < k1) totals[(uint64_t)(k + u) * lines + line] = acc;
+            acc = Op::combine(acc, v[u]);
+        }
     }
 }
 
@@ -1835,10 +1852,11 @@ __global__ __launch_bounds__(kColWaves *kWave) void col_lookback_kernel(ScanPara
 // 240 rows of 256 lines in the 16-wave tiles of col_lookback_kernel, and gives
 // a matrix four times as many chains.  Below 256 lines it replaces three
 // passes (totals, carries, rescan), 12 bytes an element instead of 8.
-// Measured on MI355X, 2^26 elements, u32 / f32, us: [2^21, 32] 139 / 141 ->
-// 85 / 111; [2^20, 64] 139 / 143 -> 85 / 105; [2^19, 128] 142 / 145 -> 89 / 99;
-// [65536, 1024] 102 / 130 -> 100 / 99; smaller, u32: [510, 659] 11.8 -> 5.4,
-// [1146, 90] 12.0 -> 5.4, [4096, 1024] 16.9 -> 8.3.
+// Measured on MI355X, 2^26 elements, u32 / f32, us: [2^21, 32] 138 / 142 ->
+// 86 / 119; [2^20, 64] 142 / 144 -> 86 / 120; [2^19, 128] 143 / 145 -> 86 / 109;
+// [65536, 1024] 102 / 130 -> 91 / 92; smaller, u32: [510, 659] 11.9 -> 5.3,
+// [1146, 90] 11.8 -> 5.6, [4096, 1024] 15.6 -> 7.2.  (f32 below 256 lines looks
+// back in order; 103, 106 and 95 for the first three without.)
 //
 // Whole 128-byte lines (row pitch and output start multiples of 128 bytes)
 // are stored non-temporally.  Elsewhere neighbouring strips share the lines
@@ -1846,8 +1864,8 @@ __global__ __launch_bounds__(kColWaves *kWave) void col_lookback_kernel(ScanPara
 // read-modify-write in memory: such strips store through the L2, and the
 // blocks are dealt so that the strips that share lines run on one XCD, whose
 // L2 then merges the parts (StripDeal).  [700001, 100] u32: 193 us
-// non-temporal, 139 through the L2, 110 with the deal (three passes: 148);
-// [165595, 486] f32 229, 185, 135 (183).
+// non-temporal, 139 through the L2, 105 with the deal (three passes: 148);
+// [165595, 486] f32 229, 185, 136 (184).
 enum StripDeal : uint32_t {
     kDealRows = 0,   // block b: strip b mod groups of chunk b / groups
     kDealChunks = 1, // every chunk's strips on one XCD, chunks round robin
@@ -1865,7 +1883,7 @@ template <int W, int STEPS> struct StripGeom {
 };
 
 // Statuses in flight per line: the f32 slots are 16 bytes, and four of them
-// a line took [2^19, 128] from 99 us to 103.
+// a line took [2^19, 128] from 99 us to 103, [8192, 256] from 9.9 to 11.0.
 template <typename T> struct StripPolls { static constexpr int value = 4; };
 template <> struct StripPolls<float> { static constexpr int value = 2; };
 
@@ -1876,14 +1894,12 @@ template <> struct StripPolls<float> { static constexpr int value = 2; };
 // chunk * lpad + entry.  A chunk that stays unpublished for p.spin_limit polls
 // is totalled from the input by the waiter, so progress never depends on the
 // dispatch order; the value is not published (every slot has one writer).
-// `base` is the line's total before the launch's first chunk, which is chunk
-// chunk0 of the axis (a scan of one launch: 0, and the identity).
-// A launch of one chunk publishes nothing (its status area is not allocated).
+// `base` is the line's total before the launch's first chunk (the identity,
+// but for a scan cut into several launches).  A launch of one chunk publishes nothing (its status area is not allocated).
 template <typename T, typename Op, typename Status, uint64_t ROWS, bool REV>
-__device__ void strip_lookback(const ScanParams &p, const Status &st, uint64_t c, uint64_t chunks, uint64_t chunk0,
-                               uint64_t lpad, uint64_t line, uint64_t entry, bool live,
-                               typename ColAcc<T>::type base, typename ColAcc<T>::type agg,
-                               typename ColAcc<T>::type &excl) {
+__device__ void strip_lookback(const ScanParams &p, const Status &st, uint64_t c, uint64_t chunks, uint64_t lpad,
+                               uint64_t line, uint64_t entry, bool live, typename ColAcc<T>::type base,
+                               typename ColAcc<T>::type agg, typename ColAcc<T>::type &excl) {
     using A = typename ColAcc<T>::type;
     constexpr int P = StripPolls<T>::value;
     if (c == 0) {
@@ -1932,7 +1948,7 @@ __device__ void strip_lookback(const ScanParams &p, const Status &st, uint64_t c
         if (live) {
             const T *in = (const T *)p.in + ((int64_t)p.in_offset + (int64_t)line);
 #pragma unroll 8
-            for (uint64_t i = (chunk0 + pos) * ROWS; i < (chunk0 + pos + 1) * ROWS; ++i) // earlier chunks are whole
+            for (uint64_t i = pos * ROWS; i < (pos + 1) * ROWS; ++i) // earlier chunks are whole
                 t = Op::combine(t, (A)in[(int64_t)(REV ? p.len - 1 - i : i) * p.in_elem_stride]);
         }
         if (!done) {
@@ -1947,19 +1963,215 @@ __device__ void strip_lookback(const ScanParams &p, const Status &st, uint64_t c
     if (live) st.publish_tile(c * lpad + entry, p.tag, kPrefix, Op::combine(excl, agg));
 }
 
+// The ordered look-back of f32 matrices below kOrderedMaxLines: results are
+// the same bits in every run.  (In the walk above an f64 sum's grouping
+// depends on the prefix that was met first.)  Chunks form groups of kStripGroup.  A chunk publishes its total, never a
+// prefix.  The last chunk of a group also publishes the group's total, and
+// then the line's total through the group, its prefix.  A chunk folds the
+// totals of its group's earlier chunks, from the first on, and then walks back
+// over whole groups, nearest first, to the first prefix and folds forward from
+// there.  So each prefix is the fold, from the left, of all group totals
+// before it, whichever prefixes the look-backs met.  A group's entries lie
+// after the chunks', (group, line) like (chunk, line).
+//
+// A status that stays unpublished for p.spin_limit polls is rebuilt by the
+// waiter with its owner's arithmetic: a chunk's total from the input, a
+// group's from its chunks.  One loop over chunks serves both: a launch fetches
+// its code cold, and with the loop in three places [240, 64] took 5.4 us
+// against 5.1.
+//
+// f32, us, first prefix met / prefixes of chunks, every total kept and folded
+// forward / groups: [16384, 64] 12.3 / 17.1 / 15.0, [524288, 64] 57.5 / 188 / 65.3,
+// [2097152, 64] 199 / 782 / 225.
+constexpr int kStripGroup = 16;
+constexpr int kStripChunkPolls = 3, kStripGroupPolls = 2; // statuses in flight per line
+
+// 64-bit words of a status.
+template <typename T> constexpr uint64_t kStripSlotWords = std::is_same<T, float>::value ? 2 : 1;
+
+template <typename T, typename Op, typename Status, int PARTS, int STEPS, bool REV>
+__device__ typename ColAcc<T>::type strip_ordered_lookback(const ScanParams &p, const Status &st, uint64_t c,
+                                                           uint64_t count, uint64_t lpad, uint64_t line,
+                                                           uint64_t entry, bool live, typename ColAcc<T>::type base,
+                                                           typename ColAcc<T>::type own) {
+    using A = typename ColAcc<T>::type;
+    const Status groups{st.words + count * lpad * kStripSlotWords<T>};
+    const A id = Op::template identity<A>();
+    if (live && count > 1) st.publish_tile(c * lpad + entry, p.tag, kAggregate, own);
+    const uint64_t g = c / kStripGroup;
+    const bool ends = c % kStripGroup == kStripGroup - 1 && c + 1 < count; // its group, with more to come
+    uint64_t lo = g * kStripGroup, hi = c; // chunks to fold
+    A before = id, through = id; // own group's total before and after this chunk
+    A prefix = id;               // the line's total through group g - 1
+    uint64_t at = g;             // group under way: back down to a prefix, then forward to g - 1
+    uint64_t found = 0;          // the group whose prefix this lane met
+    bool own_group = true, back = true, done = !live;
+    for (;;) {
+        // Fold of the totals of chunks [lo, hi), in order.
+        A sum = id;
+        uint32_t spins = 0;
+        while (lo < hi) {
+            constexpr int P = kStripChunkPolls;
+            uint32_t flag[P];
+            A val[P];
+            // Straight-line loads stay in flight together (past the end: the
+            // last one again); a wait polls one status.
+#pragma unroll
+            for (int k = 0; k < P; ++k) {
+                flag[k] = kInvalid;
+                if (k == 0 || spins == 0) st.read((lo + k < hi ? lo + k : hi - 1) * lpad + entry, p.tag, flag[k], val[k]);
+            }
+            uint32_t used = 0;
+#pragma unroll
+            for (int k = 0; k < P; ++k) {
+                if (used != (uint32_t)k || lo + k >= hi) continue;
+                if (ballot(live && flag[k] == kInvalid) != 0ull) continue;
+                sum = Op::combine(sum, val[k]);
+                used = k + 1;
+            }
+            lo += used;
+            if (used != 0) {
+                spins = 0;
+            } else if (++spins < p.spin_limit) {
+                __builtin_amdgcn_s_sleep(1);
+            } else {
+                // The total with its owner's arithmetic: each lane's STEPS
+                // rows, the lanes' totals in order.
+                A t = id;
+                if (live) {
+                    const T *in = (const T *)p.in + ((int64_t)p.in_offset + (int64_t)line);
+                    for (int e = 0; e < PARTS; ++e) {
+                        A part = id;
+#pragma unroll 4
+                        for (int k = 0; k < STEPS; ++k) {
+                            const uint64_t i = (lo * PARTS + e) * STEPS + k; // earlier chunks are whole
+                            part = Op::combine(part, (A)in[(int64_t)(REV ? p.len - 1 - i : i) * p.in_elem_stride]);
+                        }
+                        t = Op::combine(t, part);
+                    }
+                }
+                sum = Op::combine(sum, flag[0] == kInvalid ? t : val[0]);
+                ++lo;
+                spins = 0;
+            }
+        }
+        // A rebuilt value of group `at`, and whether there is one.
+        A rebuilt = id;
+        bool have = false;
+        if (own_group) {
+            own_group = false;
+            before = sum;
+            through = Op::combine(before, own);
+            if (g == 0) {
+                if (live && ends) groups.publish_tile(entry, p.tag, kPrefix, Op::combine(base, through));
+                return Op::combine(base, before);
+            }
+            if (live && ends) groups.publish_tile(g * lpad + entry, p.tag, kAggregate, through);
+            at = g - 1;
+        } else {
+            rebuilt = at == 0 ? Op::combine(base, sum) : sum;
+            have = true;
+        }
+        // Groups, until the walk ends or one has to be rebuilt.
+        spins = 0;
+        bool rebuild = false;
+        while (!rebuild) {
+            constexpr int P = kStripGroupPolls;
+            uint32_t flag[P];
+            A val[P];
+#pragma unroll
+            for (int k = 0; k < P; ++k) {
+                flag[k] = kInvalid;
+                const uint64_t u = back ? (at >= (uint64_t)k ? at - k : 0) : (at + k < g ? at + k : g - 1);
+                if (k == 0 || (spins == 0 && !have)) groups.read(u * lpad + entry, p.tag, flag[k], val[k]);
+            }
+            if (have && flag[0] == kInvalid) {
+                flag[0] = at == 0 ? kPrefix : kAggregate; // group 0 publishes only its prefix
+                val[0] = rebuilt;
+            }
+            have = false;
+            uint32_t used = 0;
+#pragma unroll
+            for (int k = 0; k < P; ++k) {
+                if (used != (uint32_t)k) continue;
+                if (back) {
+                    if (at < (uint64_t)k || ballot(!done) == 0ull) continue;
+                    if (ballot(!done && flag[k] == kInvalid) != 0ull) continue;
+                    if (!done) found = at - k;
+                    done = done || flag[k] == kPrefix;
+                } else {
+                    if (at + k >= g) continue;
+                    const bool need = live && at + k >= found;
+                    if (ballot(need && flag[k] == kInvalid) != 0ull) continue;
+                    if (need) prefix = flag[k] == kPrefix ? val[k] : Op::combine(prefix, val[k]);
+                }
+                used = k + 1;
+            }
+            if (back) {
+                if (ballot(!done) == 0ull) {
+                    // Forward from the group that the furthest lane met; with
+                    // one round the values are here.
+                    if (at == g - 1) {
+#pragma unroll
+                        for (int k = P - 1; k >= 0; --k) {
+                            if (!live || found + k > at) continue;
+                            prefix = found + k == at ? val[k] : Op::combine(prefix, val[k]);
+                        }
+                        at = g;
+                    } else {
+                        at = g - 1 - group_reduce<64>(live ? (uint32_t)(g - 1 - found) : 0u,
+                                                      [](uint32_t a, uint32_t b) { return a > b ? a : b; });
+                    }
+                    back = false;
+                    used = 1; // no wait
+                } else {
+                    at -= used;
+                }
+            } else {
+                at += used;
+            }
+            if (!back && at >= g) break;
+            if (used != 0) {
+                spins = 0;
+            } else if (++spins < p.spin_limit) {
+                __builtin_amdgcn_s_sleep(1);
+            } else {
+                rebuild = true;
+            }
+        }
+        if (!rebuild) break;
+        lo = at * kStripGroup;
+        hi = lo + kStripGroup;
+    }
+    if (live && ends) groups.publish_tile(g * lpad + entry, p.tag, kPrefix, Op::combine(prefix, through));
+    return Op::combine(prefix, before);
+}
+
 struct StripParams {
     uint32_t groups, width; // strips, lines per strip (a multiple of 4, at most W)
     uint32_t deal;          // StripDeal
     uint32_t cached;        // stores go through the L2 (else non-temporal)
     uint64_t lpad;          // status entries per chunk
     uint64_t chunks;        // of this launch
-    uint64_t chunk0;        // its first chunk's position along the axis
-    const void *totals_in;  // the lines' totals before chunk0, by entry (null: none)
-    void *totals_out;       // where the totals after the launch's last chunk go (null: nowhere)
+    uint32_t pass;          // StripPass
+    void *totals;           // a value a status entry, or (kPassTakes, kPassLeaves) two rows of them
+};
+// A launch looks back (0) or is one of three that leave the chunks' totals,
+// (col_carry_kernel in between) and start from them.  A scan cut along the
+// axis takes a launch's line totals on to the next, rows alternating.
+// PASSES launches know these forms; the others' look-back is the whole of it
+// (what they skip costs a two-chunk scan 0.4 us of cold instruction fetches:
+// [240, 100] u32 5.06 us against 4.64).
+enum StripPass : uint32_t {
+    kPassTotals = 1,  // only leave the chunks' totals
+    kPassCarries = 2, // the chunks' carries are there
+    kPassTakes = 4,   // row 0 (kPassOdd: 1) holds the lines' totals so far
+    kPassLeaves = 8,  // leave them in row 1 (kPassOdd: 0)
+    kPassOdd = 16,
 };
 
-template <typename T, typename Op, typename Status, int W, int STEPS, bool EXCL, bool REV>
-__global__ __launch_bounds__(kStripWaves *kWave) __attribute__((amdgpu_waves_per_eu(4)))
+template <typename T, typename Op, typename Status, int W, int STEPS, bool EXCL, bool REV, bool ORDERED, bool PASSES>
+__global__ __launch_bounds__(kStripWaves *kWave) __attribute__((amdgpu_waves_per_eu(ORDERED && STEPS == 8 ? 8 : 4)))
 void col_strip_kernel(ScanParams p, StripParams sp, Status st) {
     using A = typename ColAcc<T>::type;
     using G = StripGeom<W, STEPS>;
@@ -1990,6 +2202,7 @@ void col_strip_kernel(ScanParams p, StripParams sp, Status st) {
     const uint32_t cnt = p.lines - first < sp.width ? (uint32_t)(p.lines - first) : sp.width;
     const A aid = Op::template identity<A>();
 
+    const uint32_t pass = PASSES ? sp.pass : 0u;
     if (w == G::kDataWaves) {
         __syncthreads(); // the lanes' totals
         const int l = lane & (W - 1);
@@ -2002,16 +2215,30 @@ void col_strip_kernel(ScanParams p, StripParams sp, Status st) {
                 run = Op::combine(run, v);
             }
         }
-        A excl;
         const uint64_t entry = (uint64_t)g * W + l;
         const bool live = lane < (int)cnt;
-        const A base = live && sp.totals_in != nullptr ? ((const A *)sp.totals_in)[entry] : aid;
-        strip_lookback<T, Op, Status, G::kRows, REV>(p, st, c, sp.chunks, sp.chunk0, sp.lpad, first + l, entry,
-                                                     live, base, run, excl);
-        if (live && sp.totals_out != nullptr && c + 1 == sp.chunks)
-            ((A *)sp.totals_out)[entry] = Op::combine(excl, run);
+        A *totals = (A *)sp.totals;
+        if (pass & kPassTotals) {
+            if (live) totals[c * sp.lpad + entry] = run;
+            return;
+        }
+        const uint64_t odd = pass & kPassOdd ? sp.lpad : 0;
+        A excl;
+        if (pass & kPassCarries) {
+            excl = live ? totals[c * sp.lpad + entry] : aid;
+        } else {
+            A base = aid;
+            if ((pass & kPassTakes) && live) base = totals[odd + entry];
+            if constexpr (ORDERED)
+                excl = strip_ordered_lookback<T, Op, Status, G::kParts, STEPS, REV>(p, st, c, sp.chunks, sp.lpad, first + l,
+                                                                                    entry, live, base, run);
+            else
+                strip_lookback<T, Op, Status, G::kRows, REV>(p, st, c, sp.chunks, sp.lpad, first + l, entry, live, base,
+                                                             run, excl);
+        }
         if (lane < W) s_carry[l] = excl;
         __syncthreads(); // the carry
+        if ((pass & kPassLeaves) && live && c + 1 == sp.chunks) totals[sp.lpad - odd + entry] = Op::combine(excl, run);
         return;
     }
 
@@ -2023,8 +2250,8 @@ void col_strip_kernel(ScanParams p, StripParams sp, Status st) {
     const uint32_t l0 = cnt < 4 ? 0u : 4 * q + 4 <= cnt ? 4 * q : cnt - 4;
     const uint32_t nv = active ? (cnt < 4 ? cnt : 4u) : 0u;
     const uint32_t part = (uint32_t)w * G::kSub + sub;
-    const uint64_t i0 = (sp.chunk0 + c) * G::kRows + (uint64_t)part * STEPS;
-    const bool whole = (sp.chunk0 + c + 1) * G::kRows <= p.len;
+    const uint64_t i0 = c * G::kRows + (uint64_t)part * STEPS;
+    const bool whole = (c + 1) * G::kRows <= p.len;
     const T tid = Op::template identity<T>();
     T x[STEPS][4];
     {
@@ -2063,6 +2290,7 @@ void col_strip_kernel(ScanParams p, StripParams sp, Status st) {
             if ((uint32_t)v < nv) s_part[part][l0 + v] = tot[v];
     }
     __syncthreads(); // totals to the last wave
+    if (pass & kPassTotals) return;
     __syncthreads(); // its prefixes and carry
     if (!active) return;
     A run[4];
@@ -2226,8 +2454,8 @@ hx_status launch_column_v(const ScanParams &p, const ColShape &s, void *ws, hipS
     hipLaunchKernelGGL((col_totals_kernel<T, Op, V, REV>), grid, block, 0, stream, p, totals, s.chunk, s.nchunks,
                        s.groups);
     HX_TRY(check_launch("col_totals_kernel"));
-    hipLaunchKernelGGL((col_carry_kernel<A, Op>), dim3((uint32_t)ceil_div(p.lines, kWave)), dim3(kWave * kCarrySlices),
-                       0, stream, totals, p.lines, s.nchunks);
+    hipLaunchKernelGGL((col_carry_kernel<A, Op>), dim3((uint32_t)ceil_div(p.lines, kCarryLines)),
+                       dim3(kWave * kCarryWaves), 0, stream, totals, p.lines, s.nchunks);
     HX_TRY(check_launch("col_carry_kernel"));
     hipLaunchKernelGGL((col_scan_kernel<T, Op, V, EXCL, REV, true>), grid, block, 0, stream, p, (const A *)totals,
                        s.chunk, s.nchunks, s.groups);
@@ -2539,23 +2767,44 @@ constexpr uint64_t kStripDealStrips = 16;
 // [140000, 1001] - / 249 / 231, [300000, 500] - / 237 / 255.
 constexpr uint32_t kStripDealLds = 54 * 1024;
 constexpr uint64_t kStripDealManyInt = 8, kStripDealManyF32 = 16;
+// f32 matrices below this many lines give the same bits in every run: they
+// look back in order (strip_ordered_lookback), or, where the chain of chunks is
+// long and the matrix stays in the caches for a second read, take three
+// launches.  f32, us, first prefix met (other bits every run) / ordered / three
+// launches / three passes of row tiles, as it was before strips: [2048, 64] 7.0 /
+// 8.0 / - / 13.1, [4096, 64] 8.5 / 11.8 / 11.5 / 13.3, [16384, 64] 12.3 / 15.0 / 12.0 / 13.5,
+// [65536, 64] 19.0 / 22.5 / 14.9 / 13.9, [131072, 128] 30.1 / 37.3 / 43.0 / 36.1,
+// [524288, 64] 57.5 / 65.3 / 79.0 / 74.2.  Three launches always take 8 rows a
+// lane, and as many blocks to a CU as fit: they do not wait for each other.
+constexpr uint64_t kOrderedMaxLines = 256;
+constexpr uint64_t kStripCarryLen = 4096, kStripCarryMaxLen = 1ull << 18, kStripCarryElems = 1ull << 24;
 
 struct StripShape {
     int W = 64, steps = 16;
     StripParams sp{};
     uint64_t chunks = 0;   // of the axis; sp.chunks a launch
     uint64_t launches = 1;
+    bool ordered = false; // strip_ordered_lookback
+    bool carries = false; // three launches: totals, carries, rescan
     uint32_t lds = 0; // dynamic LDS, for the blocks per CU alone
 };
 
 uint64_t strip_entry_bytes(const ScanArgs &a) { return a.dtype == HX_DTYPE_F32 ? 16u : 8u; }
 uint64_t strip_total_bytes(const ScanArgs &a) { return a.dtype == HX_DTYPE_F32 ? 8u : 4u; }
+// Groups of chunks with more chunks after them, which have statuses.
+uint64_t strip_groups(const StripShape &s, uint64_t chunks) { return s.ordered ? (chunks - 1) / kStripGroup : 0; }
 // Status words of a launch, and between launches two rows of line totals
 // (read by one launch, written by the next); nothing for one chunk.
 uint64_t strip_bytes(const ScanArgs &a, const StripShape &s) {
     if (s.chunks <= 1) return 0;
-    return kLookbackOffset + s.sp.chunks * s.sp.lpad * strip_entry_bytes(a) +
+    if (s.carries) return s.chunks * s.sp.lpad * strip_total_bytes(a);
+    return kLookbackOffset + (s.sp.chunks + strip_groups(s, s.sp.chunks)) * s.sp.lpad * strip_entry_bytes(a) +
            (s.launches > 1 ? 2 * s.sp.lpad * strip_total_bytes(a) : 0);
+}
+// Rows of a chunk.
+uint64_t strip_rows(const StripShape &s) {
+    return s.steps == 8 ? (s.W == 32 ? StripGeom<32, 8>::kRows : StripGeom<64, 8>::kRows)
+                        : (s.W == 32 ? StripGeom<32, 16>::kRows : StripGeom<64, 16>::kRows);
 }
 // Blocks of a launch of `chunks` chunks.
 uint64_t strip_blocks(const StripShape &s, uint64_t chunks) {
@@ -2579,8 +2828,7 @@ StripShape strip_shape(const ScanArgs &a) {
     s.sp.lpad = (uint64_t)s.sp.groups * s.W;
     auto cut = [&](int steps) {
         s.steps = steps;
-        s.chunks = ceil_div(a.len, steps == 8 ? (s.W == 32 ? StripGeom<32, 8>::kRows : StripGeom<64, 8>::kRows)
-                                              : (s.W == 32 ? StripGeom<32, 16>::kRows : StripGeom<64, 16>::kRows));
+        s.chunks = ceil_div(a.len, strip_rows(s));
         s.sp.chunks = s.chunks;
     };
     cut(n <= kStripSmallElems && a.len <= kStripSmallLen ? 8 : 16);
@@ -2596,6 +2844,13 @@ StripShape strip_shape(const ScanArgs &a) {
             s.sp.deal = kDealStrips;
         }
     }
+    s.ordered = f32 && a.lines < kOrderedMaxLines;
+    s.carries = s.ordered && a.len > kStripCarryLen && a.len <= kStripCarryMaxLen && n < kStripCarryElems;
+    if (s.carries) {
+        cut(8);
+        s.lds = 0;
+        return s;
+    }
     // A fixed workspace too small for the statuses: 16 rows a lane halves
     // them, and what is still too long goes in several launches, each from
     // the totals the one before left.  The 8 MiB scratch, us, chunked
@@ -2605,7 +2860,8 @@ StripShape strip_shape(const ScanArgs &a) {
     if (strip_bytes(a, s) > a.workspace_limit) {
         const uint64_t row = s.sp.lpad * strip_entry_bytes(a);
         const uint64_t fixed = kLookbackOffset + 2 * s.sp.lpad * strip_total_bytes(a);
-        s.sp.chunks = a.workspace_limit > fixed ? (a.workspace_limit - fixed) / row : 0;
+        // n chunks and their groups take at most n + n / kStripGroup rows.
+        s.sp.chunks = a.workspace_limit > fixed ? (a.workspace_limit - fixed) / row * kStripGroup / (kStripGroup + 1) : 0;
         if (s.sp.chunks > kXcds) s.sp.chunks = s.sp.chunks / kXcds * kXcds;
         s.launches = s.sp.chunks > 0 ? ceil_div(s.chunks, s.sp.chunks) : 0; // 0: no room for one chunk
     }
@@ -2620,33 +2876,51 @@ bool strip_column_scan(const ScanArgs &a) {
     return s.launches > 0 && strip_blocks(s, s.sp.chunks) * (kStripWaves * kWave) <= 0xFFFFFFFFull;
 }
 
-template <typename T, typename Op, typename Status, int W, int STEPS>
+template <typename T, typename Op, typename Status, int W, int STEPS, bool ORDERED, bool PASSES>
 hx_status launch_strip_dir(const ScanParams &p, const StripShape &s, const Status &st, bool excl, bool rev,
                            hipStream_t stream) {
     const dim3 grid((uint32_t)strip_blocks(s, s.sp.chunks)), block(kStripWaves * kWave);
     if (excl && rev)
-        hipLaunchKernelGGL((col_strip_kernel<T, Op, Status, W, STEPS, true, true>), grid, block, s.lds, stream, p, s.sp,
-                           st);
+        hipLaunchKernelGGL((col_strip_kernel<T, Op, Status, W, STEPS, true, true, ORDERED, PASSES>), grid, block, s.lds,
+                           stream, p, s.sp, st);
     else if (excl)
-        hipLaunchKernelGGL((col_strip_kernel<T, Op, Status, W, STEPS, true, false>), grid, block, s.lds, stream, p,
-                           s.sp, st);
+        hipLaunchKernelGGL((col_strip_kernel<T, Op, Status, W, STEPS, true, false, ORDERED, PASSES>), grid, block, s.lds,
+                           stream, p, s.sp, st);
     else if (rev)
-        hipLaunchKernelGGL((col_strip_kernel<T, Op, Status, W, STEPS, false, true>), grid, block, s.lds, stream, p,
-                           s.sp, st);
+        hipLaunchKernelGGL((col_strip_kernel<T, Op, Status, W, STEPS, false, true, ORDERED, PASSES>), grid, block, s.lds,
+                           stream, p, s.sp, st);
     else
-        hipLaunchKernelGGL((col_strip_kernel<T, Op, Status, W, STEPS, false, false>), grid, block, s.lds, stream, p,
-                           s.sp, st);
+        hipLaunchKernelGGL((col_strip_kernel<T, Op, Status, W, STEPS, false, false, ORDERED, PASSES>), grid, block,
+                           s.lds, stream, p, s.sp, st);
     return check_launch("col_strip_kernel");
+}
+
+template <typename T, typename Op, typename Status, int W, bool ORDERED>
+hx_status launch_strip_steps(const ScanParams &p, const StripShape &s, const Status &st, bool excl, bool rev,
+                             hipStream_t stream) {
+    // Several launches: three (ordered), or 16 rows a lane below 256 lines.
+    constexpr bool kMayPass8 = ORDERED, kMayPass16 = ORDERED || !std::is_same<T, float>::value;
+    const bool passes = s.carries || s.launches > 1;
+    if (s.steps == 8) {
+        if constexpr (kMayPass8)
+            if (passes) return launch_strip_dir<T, Op, Status, W, 8, ORDERED, true>(p, s, st, excl, rev, stream);
+        if (!passes) return launch_strip_dir<T, Op, Status, W, 8, ORDERED, false>(p, s, st, excl, rev, stream);
+    } else {
+        if constexpr (kMayPass16)
+            if (passes) return launch_strip_dir<T, Op, Status, W, 16, ORDERED, true>(p, s, st, excl, rev, stream);
+        if (!passes) return launch_strip_dir<T, Op, Status, W, 16, ORDERED, false>(p, s, st, excl, rev, stream);
+    }
+    return fail(HX_ERR_DISPATCH_FAILED, "a column scan of this shape takes one launch");
 }
 
 template <typename T, typename Op, typename Status>
 hx_status launch_strip_shaped(const ScanParams &p, const StripShape &s, const Status &st, bool excl, bool rev,
                               hipStream_t stream) {
-    if (s.W == 32)
-        return s.steps == 8 ? launch_strip_dir<T, Op, Status, 32, 8>(p, s, st, excl, rev, stream)
-                            : launch_strip_dir<T, Op, Status, 32, 16>(p, s, st, excl, rev, stream);
-    return s.steps == 8 ? launch_strip_dir<T, Op, Status, 64, 8>(p, s, st, excl, rev, stream)
-                        : launch_strip_dir<T, Op, Status, 64, 16>(p, s, st, excl, rev, stream);
+    constexpr bool kMayOrder = std::is_same<T, float>::value; // strips of 32 lines are always ordered there
+    if (s.W == 32) return launch_strip_steps<T, Op, Status, 32, kMayOrder>(p, s, st, excl, rev, stream);
+    if constexpr (kMayOrder)
+        if (s.ordered) return launch_strip_steps<T, Op, Status, 64, true>(p, s, st, excl, rev, stream);
+    return launch_strip_steps<T, Op, Status, 64, false>(p, s, st, excl, rev, stream);
 }
 
 template <typename T, typename Op>
@@ -2656,18 +2930,38 @@ hx_status launch_strip(const ScanArgs &a, ScanParams p, void *ws, uint64_t ws_by
     if (ws_bytes < strip_bytes(a, s))
         return fail(HX_ERR_DISPATCH_FAILED, "scan workspace of %llu bytes is too small", (unsigned long long)ws_bytes);
     uint64_t *words = (uint64_t *)((char *)ws + kLookbackOffset);
-    char *totals = (char *)words + s.sp.chunks * s.sp.lpad * strip_entry_bytes(a);
-    const uint64_t row = s.sp.lpad * strip_total_bytes(a), per = s.sp.chunks;
-    for (uint64_t k = 0; k < s.launches; ++k) {
-        s.sp.chunk0 = k * per;
-        s.sp.chunks = std::min(per, s.chunks - s.sp.chunk0);
-        s.sp.totals_in = k > 0 ? totals + (k % 2) * row : nullptr;
-        s.sp.totals_out = k + 1 < s.launches ? totals + ((k + 1) % 2) * row : nullptr;
-        if (s.chunks > 1) HX_TRY(next_lookback_launch(lb, ws, ws_bytes, stream, &p.tag));
+    auto launch = [&] {
         if constexpr (std::is_same<T, float>::value)
-            HX_TRY((launch_strip_shaped<T, Op>(p, s, F64QuadDense{words}, a.exclusive, a.reverse, stream)));
+            return launch_strip_shaped<T, Op>(p, s, F64QuadDense{words}, a.exclusive, a.reverse, stream);
         else
-            HX_TRY((launch_strip_shaped<T, Op>(p, s, PackedStatus{words}, a.exclusive, a.reverse, stream)));
+            return launch_strip_shaped<T, Op>(p, s, PackedStatus{words}, a.exclusive, a.reverse, stream);
+    };
+    if (s.carries) {
+        using A = typename ColAcc<T>::type;
+        s.sp.totals = ws;
+        s.sp.pass = kPassTotals;
+        HX_TRY(launch());
+        hipLaunchKernelGGL((col_carry_kernel<A, Op>), dim3((uint32_t)ceil_div(s.sp.lpad, kCarryLines)),
+                           dim3(kWave * kCarryWaves), 0, stream, (A *)ws, s.sp.lpad, (uint32_t)s.chunks);
+        HX_TRY(check_launch("col_carry_kernel"));
+        s.sp.pass = kPassCarries;
+        return launch();
+    }
+    const uint64_t per = s.sp.chunks, rows = strip_rows(s);
+    s.sp.totals = (char *)words + (per + strip_groups(s, per)) * s.sp.lpad * strip_entry_bytes(a);
+    for (uint64_t k = 0; k < s.launches; ++k) {
+        // Launch k scans what the earlier ones left of the lines (a mirrored
+        // line's end is its far end: the offsets stay).
+        const uint64_t done = k * per * rows;
+        p.len = a.len - done;
+        if (!a.reverse) {
+            p.in_offset = a.in_offset + (uint64_t)((int64_t)done * a.in_elem_stride);
+            p.out_offset = a.out_offset + (uint64_t)((int64_t)done * a.out_elem_stride);
+        }
+        s.sp.chunks = std::min(per, s.chunks - k * per);
+        s.sp.pass = (k > 0 ? kPassTakes : 0u) | (k + 1 < s.launches ? kPassLeaves : 0u) | (k % 2 ? kPassOdd : 0u);
+        if (s.chunks > 1) HX_TRY(next_lookback_launch(lb, ws, ws_bytes, stream, &p.tag));
+        HX_TRY(launch());
         if (s.chunks > 1) commit_lookback_launch(lb);
     }
     return HX_OK;
@@ -2821,7 +3115,8 @@ uint64_t scan_fixed_workspace_bytes(const ScanArgs &a) { return fixed_workspace_
 
 bool scan_uses_lookback(const ScanArgs &a) {
     if (short_line_scan(a)) return false;
-    if (rowtile_column_scan(a) || strip_column_scan(a)) return scan_bytes(a) > 0; // one tile or chunk: none
+    if (rowtile_column_scan(a)) return scan_bytes(a) > 0; // one tile: none
+    if (strip_column_scan(a)) return scan_bytes(a) > 0 && !strip_shape(a).carries; // one chunk: none
     return !column_mode(a) || column_single_pass(a);
 }
 

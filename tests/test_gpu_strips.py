@@ -94,6 +94,41 @@ def test_strip_scan_under_forced_fallbacks(device, oracle, limits, dtype, rows, 
         check(device, oracle, rows, cols, dtype, seed=rows, reverse=reverse, exclusive=reverse)
 
 
+# f32 values over 46 powers of two, the second half of the rows the negated
+# first in another order, so that the last outputs are what the f64 sums
+# rounded: any other order of the chunk totals shows in the bits.
+def _rounding_sensitive(rows, cols, pitch, offset):
+    rng = np.random.default_rng(rows + cols)
+    half = rows // 2
+    x = np.zeros((rows, pitch), np.float32)
+    x[:half] = (rng.uniform(-1, 1, (half, pitch)) * np.exp2(rng.integers(0, 46, (half, pitch)))).astype(np.float32)
+    x[half:2 * half] = -x[rng.permutation(half)]
+    return np.concatenate([np.zeros(offset, np.float32), x.ravel()])
+
+
+@pytest.mark.parametrize("rows,cols,pitch,offset,exclusive,reverse", [
+    (8_192, 32, 32, 0, False, False), (7_001, 45, 47, 3, True, False), (50_000, 64, 64, 0, False, True),
+    (60_000, 100, 100, 0, True, True), (8_193, 255, 255, 1, False, False), (700_000, 33, 33, 0, False, True),
+    (400_000, 64, 64, 0, True, False), (200_000, 130, 131, 0, False, False)])
+def test_f32_strips_below_256_lines_give_the_same_bits_in_every_run(device, oracle, rows, cols, pitch, offset, exclusive, reverse):
+    lay = Layout.try_new([rows, cols], [pitch, 1], offset)
+    x = device.upload(_rounding_sensitive(rows, cols, pitch, offset))
+    out = device.alloc_zeroed(np.float32, offset + rows * pitch)
+
+    def run():
+        SCAN.scan_axis_into(device, hx.CumSumOp, StridedView(x, lay), 0,
+                            hx.ScanDirection.Reverse if reverse else hx.ScanDirection.Forward, StridedView(out, lay),
+                            hx.ScanKind.Exclusive if exclusive else hx.ScanKind.Inclusive)
+        return device.download_owned(out).view(np.uint32)
+
+    first = run()
+    for _ in range(10):
+        assert np.array_equal(run(), first)
+    for limits in ((0, 0), (1, 1)):  # waiters total missing chunks themselves
+        with wait_limits(*limits):
+            assert np.array_equal(run(), first), limits
+
+
 # Taken by the fixed scratch, but with more status words than it holds as
 # strips are first cut: [94200, 1279] takes longer chunks, the others several
 # launches, each from the totals of the one before.  Rows at multiples of
