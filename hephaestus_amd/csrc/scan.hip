@@ -2523,8 +2523,10 @@ struct TileShape {
 // f32 lines took 12 x 16 tiles (one block per CU) before f32 tiles fit in
 // 128 VGPRs; 8 x 16 at two blocks per CU: 2^30 f32 1373.1 -> 1315.6 us.
 constexpr int kLongWaves = 8, kLongSteps = 16;
-// Few lines of more than 2048 elements leave most of the chip idle in tiles
-// that large: a block moves its 128 KiB at one CU's rate, and 2^20 elements
+// Few lines of more than 4096 elements leave most of the chip idle in tiles
+// that large (up to 4096 one tile is as fast as a chain or faster: u32 lines of
+// 3000 elements 3.2 us against 3.7, 3 lines of 4096 3.3 against 3.8): a block
+// moves its 128 KiB at one CU's rate, and 2^20 elements
 // are 32 blocks.  Fewer than 256 lines take smaller tiles and chain them,
 // while the tiles number about four or five a CU: 2048 elements up to 2^17,
 // 4096 up to 2^22, 8192 up to kMid8192Elems (2^23 where the outputs do not
@@ -2536,7 +2538,7 @@ constexpr int kLongWaves = 8, kLongSteps = 16;
 // Chained tiles have status words.  Where a launch of its own clears them
 // (ScanArgs::clears) a line that one tile holds keeps it up to kClearOneTile
 // elements, and beyond where it fills the tile: a graph node of u32 lines of
-// 2049 / 8192 / 32768 elements 3.1 / 3.1 / 5.1 us against 5.3 / 5.1 / 5.3 for clear
+// 5000 / 8192 / 32768 elements 4.1 / 3.1 / 5.1 us against 5.3 / 5.1 / 5.3 for clear
 // and scan, but 12000 6.2 against 5.2 (a tile that is not full loads element
 // by element).
 constexpr uint64_t kMidMaxLines = 255;
@@ -2557,11 +2559,11 @@ inline TileShape tile_shape(const ScanArgs &a) {
     const uint64_t len = a.len, n = a.len * a.lines;
     const TileShape one = line_tile_shape(len);
     const bool keep_one = a.clears && len <= one.elems() && (len <= kClearOneTile || len == one.elems());
-    if (len > 2048 && !keep_one && a.lines <= kMidMaxLines && a.in_elem_stride == 1 && a.out_elem_stride == 1) {
+    if (len > 4096 && !keep_one && a.lines <= kMidMaxLines && a.in_elem_stride == 1 && a.out_elem_stride == 1) {
         const bool grid = ((uintptr_t)a.out + 4u * a.out_offset + (a.reverse ? 4u * len : 0u)) % 128 == 0;
         if (n <= kMid2048Elems) return {2, 4};
         if (n <= kMid4096Elems) return {4, 4};
-        if (len > 4096 && n <= (grid ? kMid8192Elems : 1ull << 23)) return {4, 8};
+        if (n <= (grid ? kMid8192Elems : 1ull << 23)) return {4, 8};
     }
     return one;
 }
