@@ -901,6 +901,8 @@ struct Shape {
 //     more than wider loads gain, 33 x 2049 2.8 / 3.5, 256 x 301 3.3 / 3.8, until
 //     a last group of a few outputs fetches its lines almost alone, 700 x 65
 //     5.5 / 4.4, 1024 x 257 6.2 / 4.7.
+//   more than kSliceLines lines: a wave's slice of single outputs is long, 1000
+//     x 30 5.0 / 4.3, 1024 x 301 4.5 / 4.5; but u32 700 x 30 3.9 / 4.0.
 //   beyond that many elements, up to kBlockFoldLines lines: 256 x 10241 6.6 / 3.8.
 //   more lines: a wave of vectors has few lanes at few outputs, 10^6 x 11
 //     (padded) 22 / 78, 6000 x 201 6.0 / 6.8, 100000 x 193 17.5 / 21.5.  Vectors
@@ -908,7 +910,7 @@ struct Shape {
 //     with many lines, 6000 x 1001 9.7 / 8.8, 4096 x 1001 6.9 / 7.9.
 constexpr uint64_t kVectorWide = 1ull << 18;
 constexpr uint64_t kVectorMinCols = 640, kVectorMinLines = 5000, kVectorElems = 3ull << 23;
-constexpr uint64_t kLastGroup = 8, kLastGroupLines = 256;
+constexpr uint64_t kLastGroup = 8, kLastGroupLines = 256, kSliceLines = 768;
 bool column_vectors(const RowParams &p, uintptr_t base) {
     if (p.row_stride != 1 || p.rows < 4 || base % 4 != 0) return false;
     if (p.rows % 4 == 0) return true;
@@ -916,7 +918,8 @@ bool column_vectors(const RowParams &p, uintptr_t base) {
     if (lines <= kMinColChunk) return outputs >= kVectorWide;
     if (lines <= kBlockFoldLines) {
         const uint64_t last = outputs % kWave;
-        return outputs * lines > kBlockFoldElems || (lines > kLastGroupLines && last > 0 && last <= kLastGroup);
+        return outputs * lines > kBlockFoldElems || lines > kSliceLines ||
+               (lines > kLastGroupLines && last > 0 && last <= kLastGroup);
     }
     return outputs >= kBlockManyCols || (outputs >= kVectorMinCols && lines >= kVectorMinLines) ||
            (outputs >= 2 * kWave && outputs * lines >= kVectorElems);
