@@ -2412,21 +2412,40 @@ bool column_short_lines(const ScanArgs &a) {
     const ColShape s = column_shape(a);
     return s.nchunks == 1 && a.len <= kColShortMaxLen && s.groups >= kColShortMinGroups;
 }
-// Large integer matrices keep col_lookback_kernel's 1 KiB rows against the
-// strips' 256 bytes, from 1024 lines where the rows are whole 128-byte lines
-// and from 4096 where they are whole 16-byte vectors: u32, us, [32768, 4096]
-// 182 against 195, [131072, 1024] 189 against 201, [49152, 2048] 146 against
-// 153, [26541, 4532] 205 against 211; but [524288, 256] 250 against 200, [65536,
-// 1024] 102 against 91, [30000, 5001] 275 against 267.
+// Where col_lookback_kernel's 1 KiB rows beat the strips' 256 bytes:
+//   Large integer matrices from 1024 lines where the rows are whole 128-byte
+//   lines and from 4096 where they are whole 16-byte vectors: u32, us, rows of
+//   1 KiB / strips: [32768, 4096] 182 / 195, [131072, 1024] 189 / 201, [49152,
+//   2048] 146 / 153, [26541, 4532] 205 / 211; but [524288, 256] 250 / 200, [65536,
+//   1024] 102 / 91.
+//   Matrices beyond the caches whose strips share 128-byte lines, from 8192
+//   lines: u32 / f32, us, [2048, 50001] 189 / 238, [4096, 32001] 242 / 338 and 250 /
+//   323, [512, 200001] 184 / 234 and 197 / 239; more lines have few rows, and f32
+//   strips keep those: [400, 300001] u32 231 / 286, [300, 400001] f32 252 / 196.
+//   One round of blocks, one to a CU, with half their rows or more: u32 / f32,
+//   us, [240, 65536] 19.0 / 24.4 and 20.3 / 26.7, [200, 50001] 17.0 / 20.0 and 18.1 /
+//   20.2, but [128, 50001] 11.3 / 12.4 and 12.6 / 11.8; two rounds of whole lines that
+//   nearly fill the chip: u32 [300, 65536] 27.9 / 34.4, f32 [480, 65536] 44.7 / 56.1,
+//   but [350, 40000] u32 21.9 / 20.9.
 constexpr uint64_t kWideLines = 1024, kWideVectorLines = 4096;
 constexpr uint64_t kWideElems = 1ull << 26;
+constexpr uint64_t kWideSharedLines = 8192, kWideSharedMaxInt = 1ull << 19, kWideSharedMaxF32 = 1ull << 18;
+constexpr uint64_t kWideSharedElemsInt = 5ull << 24, kWideSharedElemsF32 = 3ull << 25;
+constexpr uint64_t kWideBlocks = 256, kWideRoundElems = 1ull << 23;
 bool whole_line_rows(const ScanArgs &a) {
     return ((uintptr_t)a.out + 4u * a.out_offset) % 128 == 0 && a.out_elem_stride % 32 == 0; // 4-byte elements
 }
 bool column_wide(const ScanArgs &a) {
-    if (a.dtype == HX_DTYPE_F32 || a.len * a.lines <= kWideElems) return false;
-    return (a.lines >= kWideLines && whole_line_rows(a)) ||
-           (a.lines >= kWideVectorLines && a.out_elem_stride % 4 == 0);
+    const uint64_t n = a.len * a.lines;
+    const bool f32 = a.dtype == HX_DTYPE_F32, whole = whole_line_rows(a);
+    const ColLbShape s = col_lb_shape(a);
+    if (s.groups <= kWideBlocks && s.chunks <= 2 && n > s.chunks * kWideRoundElems)
+        return s.chunks == 1 || (whole && s.groups > kWideBlocks * 3 / 4);
+    if (!whole && a.lines >= kWideSharedLines && a.lines <= (f32 ? kWideSharedMaxF32 : kWideSharedMaxInt) &&
+        n > (f32 ? kWideSharedElemsF32 : kWideSharedElemsInt))
+        return true;
+    if (f32 || n <= kWideElems) return false;
+    return (a.lines >= kWideLines && whole) || (a.lines >= kWideVectorLines && a.out_elem_stride % 4 == 0);
 }
 bool column_single_pass(const ScanArgs &a) {
     return column_mode(a) && a.lines >= kSinglePassMinLines && !column_short_lines(a) &&
@@ -2485,7 +2504,8 @@ hx_status launch_col_lookback(const ScanParams &p, const ColLbShape &s, bool exc
     if constexpr (std::is_same<T, float>::value) {
         // Ascending f32 lines take the strips (column_single_pass).
         const F64PairStatus st{(uint64_t *)status};
-        return launch_col_lookback_s<T, Op, F64PairStatus, 1>(p, s, st, excl, rev, stream);
+        return s.V == 4 ? launch_col_lookback_s<T, Op, F64PairStatus, 4>(p, s, st, excl, rev, stream)
+                        : launch_col_lookback_s<T, Op, F64PairStatus, 1>(p, s, st, excl, rev, stream);
     } else {
         const PackedStatus st{(uint64_t *)status};
         return s.V == 4 ? launch_col_lookback_s<T, Op, PackedStatus, 4>(p, s, st, excl, rev, stream)
@@ -2745,8 +2765,12 @@ hx_status launch_rowtile_lb(const ScanArgs &a, ScanParams p, void *ws, uint64_t 
 //
 // Rows per lane: 16, and 8 where the matrix is small and its chains stay
 // short (u32, us, 8 / 16 rows: [510, 659] 5.2 / 6.4, [16384, 512] 12.8 / 14.5,
-// [8192, 2048] 26.5 / 28.2, but [100000, 64] 17.5 / 15.5) and where many strips
-// share lines (below).
+// [8192, 2048] 26.5 / 28.2, but [100000, 64] 17.5 / 15.5), where many strips share
+// lines (below), and where 8 rows a lane hold the lines and 16 would leave
+// waves without a row (f32, us, 8 / 16 rows: [40, 1000001] 68 / 147, [72, 400001]
+// 43 / 69, [128, 200001] 41 / 48); beyond the caches only up to half of them
+// ([224, 400001] 194 / 153).
+constexpr uint64_t kStripOneChunk = StripGeom<64, 8>::kRows;
 constexpr uint64_t kStripSmallElems = 1ull << 24;
 constexpr uint64_t kStripSmallLen = 1ull << 16;
 // Stores of whole lines that go through the L2 all the same: sizes from
@@ -2833,7 +2857,9 @@ StripShape strip_shape(const ScanArgs &a) {
         s.chunks = ceil_div(a.len, strip_rows(s));
         s.sp.chunks = s.chunks;
     };
-    cut(n <= kStripSmallElems && a.len <= kStripSmallLen ? 8 : 16);
+    const bool small = n <= kStripSmallElems && a.len <= kStripSmallLen;
+    const bool few_rows = a.len <= kStripOneChunk && (a.len <= kStripOneChunk / 2 || n <= kStripCachedElems);
+    cut(small || few_rows ? 8 : 16);
     const bool lines128 = whole_line_rows(a) && s.sp.width % 32 == 0;
     s.sp.cached = !lines128 || (s.sp.groups > 1 && n > kStripSmallElems && n <= kStripCachedElems) ? 1u : 0u;
     s.sp.deal = kDealRows;
