@@ -129,9 +129,12 @@ hx_status launch_clear_words(void *words, uint64_t count, hipStream_t stream) {
 
 hx_status launch_read_back(const void *src, void *dst, uint32_t bytes, uint64_t *flag, uint64_t sequence,
                            hipStream_t stream) {
-    hipLaunchKernelGGL(read_back_kernel, dim3(1), dim3(kReadBackBlock), 0, stream, (const uint8_t *)src, (uint8_t *)dst,
-                       bytes, flag, sequence);
-    return check_launch("read_back_kernel");
+    // The launch's own status: the thread's last error may be an earlier
+    // call's, and says nothing about this download.
+    void *args[] = {&src, &dst, &bytes, &flag, &sequence};
+    HX_HIP(hipLaunchKernel((const void *)read_back_kernel, dim3(1), dim3(kReadBackBlock), args, 0, stream),
+           HX_ERR_TRANSFER_FAILED, "read_back_kernel");
+    return HX_OK;
 }
 
 hx_status launch_copy_scan_shape(const void *src, void *dst, uint64_t bytes, hipStream_t stream) {

@@ -1,5 +1,6 @@
 """Small downloads: sizes around the pinned slots' and a word's, odd addresses,
-results of kernels queued just before, and more threads than slots."""
+results of kernels queued just before, long queues, an error left by an earlier
+call, and more threads than slots."""
 from __future__ import annotations
 
 import threading
@@ -9,6 +10,8 @@ import pytest
 
 import hephaestus_amd as hx
 from hephaestus_amd import _ffi
+
+from test_gpu_capture import _hip
 
 pytestmark = pytest.mark.gpu
 
@@ -36,18 +39,47 @@ def test_sees_work_queued_before(device):
         assert device.download_owned(b)[-1] == (2.0 if k % 2 else 1.0)
 
 
+def test_waits_for_long_queued_work(device):
+    """Milliseconds of queued work: longer than the host watches the flag."""
+    n = 1 << 28
+    x, y = device.alloc_zeroed(np.uint32, n), device.alloc_zeroed(np.uint32, n)
+    device.write_sub_buffer(x, 0, np.array([7], np.uint32))
+    lay = hx.Layout.c_contiguous([n])
+    tail = np.zeros(3, np.uint32)
+    for k, (src, dst) in enumerate([(x, y), (y, x), (x, y)]):
+        for _ in range(4):
+            hx.RocmScanOps().scan_axis_into(device, hx.CumSumOp, hx.StridedView(src, lay), 0, hx.ScanDirection.Forward,
+                                            hx.StridedView(dst, lay), hx.ScanKind.Inclusive)
+        _ffi.check(_ffi.lib().hx_download(device.handle, dst.ptr + 4 * (n - 3), 3, tail.ctypes.data, 3, 4))
+        want = np.arange(n - 2, n + 1, dtype=np.uint64)
+        want = [7 * np.ones(3, np.uint64), 7 * want, 7 * want * (want + 1) // 2][k]
+        assert np.array_equal(tail, want.astype(np.uint32)), k
+    x.free()
+    y.free()
+
+
+def test_an_earlier_error_of_the_thread_is_not_the_downloads(device):
+    host = np.arange(5, dtype=np.uint32)
+    buffer = device.upload(host)
+    assert _hip().hipSetDevice(999) != 0
+    try:
+        got = device.download_owned(buffer)
+    finally:
+        _hip().hipGetLastError()
+    assert np.array_equal(got, host)
+
+
 def test_more_threads_than_slots(device):
     buffers = [device.upload(np.arange(17, dtype=np.uint32) + 1000 * t) for t in range(20)]
-    wrong = []
+    right = [0] * len(buffers)
 
     def work(t):
         for _ in range(100):
-            if not np.array_equal(device.download_owned(buffers[t]), np.arange(17, dtype=np.uint32) + 1000 * t):
-                wrong.append(t)
+            right[t] += np.array_equal(device.download_owned(buffers[t]), np.arange(17, dtype=np.uint32) + 1000 * t)
 
     threads = [threading.Thread(target=work, args=(t,)) for t in range(len(buffers))]
     for t in threads:
         t.start()
     for t in threads:
         t.join()
-    assert not wrong
+    assert right == [100] * len(buffers)  # a download that raised ends its thread
