@@ -370,19 +370,17 @@ def run_column_scan(device, oracle, op, dtype, shape, strides, offset, axis, exc
             assert np.array_equal(g, w)
 
 
-# (rows, cols) scanned along axis 0.  Single-pass look-back (256 lines and
-# more): 16-byte lanes over many chunks, line counts 3, 1 and 2 past a
-# multiple of 4 (the last group's lane moves its lines one by one), one tile
-# only; the chunked form with 130 lines.
+# (rows, cols) scanned along axis 0 in strips: many chunks, line counts 3, 1
+# and 2 past a multiple of 4 (a strip's last lane moves back to a whole
+# vector), one chunk only.
 COLUMN_SHAPES = [(4099, 1000), (3001, 999), (3001, 1001), (2000, 1022), (20, 256), (5000, 130),
-                 # narrow columns (32, 64, 128): the dense range scanned with
-                 # strided lane scans, one or many chunks
+                 # one or two whole strips
                  (4097, 32), (1000, 64), (3001, 128),
-                 # other columns below 256: row tiles of up to 16384 elements
-                 # staged through LDS, a thread per column and row group.  Up
-                 # to 24 columns one pass with a look-back over C-wide carries
-                 # (257 tiles for 2 and 4 columns), wider three passes; many
-                 # tiles with a partial last one, a single tile, one row
+                 # up to 24 columns: row tiles of up to 16384 elements staged
+                 # through LDS, a thread per column and row group, with a
+                 # look-back over C-wide carries (257 tiles for 2 and 4
+                 # columns); many tiles with a partial last one, a single
+                 # tile, one row; 100 to 255 columns strips again
                  ((1 << 20) + 1, 2), ((1 << 20) + 3, 4), (70001, 3), (30001, 5), (4099, 7), (70001, 8),
                  (20001, 12), (65536, 16), (5000, 24), (3000, 100), (1000, 200), (3001, 255), (5, 3), (5, 4),
                  (1, 6)]
@@ -476,7 +474,7 @@ def test_row_scan_tile_shapes(device, oracle, shape, dtype, variant):
 @pytest.mark.parametrize("shape", [(3001, 1000), (3000, 100), (100003, 8), (100003, 3), (30001, 6)])
 def test_column_scan_off_16_byte_boundaries(device, oracle, shape, dtype):
     # offset 1: every line's vectors start 4 bytes past a 16-byte boundary
-    # (single pass for 1000 lines, row tiles for the others); vectors need only 4-byte
+    # (strips for 100 and 1000 lines, row tiles for the others); vectors need only 4-byte
     # alignment, so both keep one 16-byte access per lane and step
     r, c = shape
     run_column_scan(device, oracle, "sum", dtype, shape, (c, 1), 1, 0, False, False, seed=r + c)
@@ -490,8 +488,7 @@ def test_column_scan_off_16_byte_boundaries(device, oracle, shape, dtype):
 @pytest.mark.parametrize("shape,ld", [((3000, 100), 104), ((65536, 16), 17)])
 def test_chunked_column_scan_of_padded_rows(device, oracle, shape, ld, dtype, op, reverse, kind):
     # rows padded past their width (line stride 1, element stride ld > C):
-    # not the dense range of the row-tile or narrow forms, so fewer than 256
-    # lines take the chunked reduce-then-scan
+    # not the dense range of the row tiles, so these widths take strips too
     r, c = shape
     run_column_scan(device, oracle, op, dtype, shape, (ld, 1), 0, 0, kind == "exclusive", reverse, seed=r + ld)
 
@@ -548,9 +545,9 @@ def test_prepared_axis_reduction_batch(device, oracle):
 @pytest.mark.parametrize("reverse", [False, True])
 @pytest.mark.parametrize("c", [32, 8, 100])
 def test_prepared_narrow_column_scan_rebinds(device, oracle, reverse, c):
-    # narrow-column scans through a prepared plan (narrow form, one-pass and
-    # three-pass row tiles): the workspace for the carries or look-back
-    # statuses comes with the plan; later writes to the input are observed
+    # narrow-column scans through a prepared plan (strips of 32 and 64 lines,
+    # row tiles): the workspace for the look-back statuses comes with the
+    # plan; later writes to the input are observed
     r = 300001
     lay = Layout.c_contiguous([r, c])
     x = oracle.uniform_int(r * c, seed=4, lo=0, hi=1000)

@@ -118,9 +118,9 @@ def test_scans_under_forced_fallbacks(device, oracle, limits, exclusive, reverse
     assert bad == 0, worst
 
 
-# Single-pass column look-back (256 lines and more): integer and f32 lines,
-# sums and products, forward and reverse; 1003 lines leave a partial last
-# group, whose rebuilt aggregates read only the lines that exist.
+# Strips of column scans: integer and f32 lines, sums and products, forward
+# and reverse; 1003 lines leave a partial last strip, whose rebuilt totals
+# read only the lines that exist.
 @pytest.mark.parametrize("limits", FORCED)
 @pytest.mark.parametrize("dtype", [np.uint32, np.float32])
 @pytest.mark.parametrize("reverse", [False, True])
@@ -131,9 +131,10 @@ def test_column_lookback_scans_under_forced_fallbacks(device, oracle, limits, dt
         run_column_scan(device, oracle, "sum", dtype, (2001, 1003), (1003, 1), 0, 0, True, reverse, seed=21)
 
 
-# Row-tile column look-back (axis 0 of dense matrices with 2 to 255 columns
-# outside the narrow form): a missing predecessor's column aggregate is
-# rebuilt from the input by the waiting thread.  13, 15 and 47 tiles.
+# Row-tile column look-back (axis 0 of dense matrices with 2 to 24 columns):
+# a missing predecessor's column aggregate is rebuilt from the input by the
+# waiting thread.  13 and 15 tiles; 255 columns are strips in f32's fixed
+# order.
 @pytest.mark.parametrize("limits", FORCED)
 @pytest.mark.parametrize("dtype", [np.uint32, np.float32])
 @pytest.mark.parametrize("reverse", [False, True])

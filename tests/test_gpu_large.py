@@ -181,8 +181,8 @@ def test_rows_past_2_31_rows(device):
 
 @pytest.mark.parametrize("kind,reverse", [("inclusive", False), ("exclusive", True)])
 def test_narrow_column_scan_with_many_tiles(device, kind, reverse):
-    """[2^23 + 5, 64] u32 along axis 0: 10923 tiles of 12288 vectors, so
-    each thread of the carry pass owns 11 tiles (past its one-batch case).
+    """[2^23 + 5, 64] u32 along axis 0: one strip of 18725 chunks of 448 rows,
+    each looking back along the strip.
     Every element is 1 except x[r0][c0] = 1000, so column c gets out[r][c] =
     r + 1 (inclusive forward) or R - 1 - r (exclusive reverse), plus 999 in
     column c0 from row r0 on (forward) or before row r0 (reverse)."""
@@ -196,7 +196,7 @@ def test_narrow_column_scan_with_many_tiles(device, kind, reverse):
     SCAN.scan_axis_into(device, hx.CumSumOp, StridedView(x, lay), 0,
                         hx.ScanDirection.Reverse if reverse else hx.ScanDirection.Forward, StridedView(out, lay),
                         hx.ScanKind.Exclusive if kind == "exclusive" else hx.ScanKind.Inclusive)
-    for r in (0, 1, 767, 768, r0 - 1, r0, r0 + 1, (1 << 23) - 1, R - 1):  # 768 rows per tile
+    for r in (0, 1, 767, 768, r0 - 1, r0, r0 + 1, (1 << 23) - 1, R - 1):
         got = _slice(device, out, r * C, C)
         want = np.full(C, (R - 1 - r) if reverse else (r + 1), np.uint64)
         if (r < r0) if reverse else (r >= r0):
@@ -209,11 +209,9 @@ def test_narrow_column_scan_with_many_tiles(device, kind, reverse):
 @pytest.mark.parametrize("kind,reverse", [("inclusive", False), ("exclusive", True)])
 @pytest.mark.parametrize("C,R,tile_rows", [(3, 3 * (1 << 24) + 5, 5440), (100, 1500007, 160)])
 def test_row_tile_column_scan_with_many_tiles(device, kind, reverse, C, R, tile_rows):
-    """Row tiles along axis 0, u32, with about 9200 tiles: [3 * 2^24 + 5, 3]
-    (tiles of 5440 rows, whole 128-byte lines) looks back in one pass over
-    9253 tiles;
-    [1500007, 100] (tiles of 160 rows, 9376 tiles) takes three passes, and
-    each thread of its carry pass owns 10 tiles (past its one-batch case).
+    """Long look-backs along axis 0, u32: [3 * 2^24 + 5, 3] over 9253 row tiles
+    (of 5440 rows, whole 128-byte lines), [1500007, 100] over strips of 52 and
+    48 lines in chunks of 448 rows (sampled every 160 rows).
     Every element is 1 except x[r0][c0] = 1000, as in the narrow case
     above."""
     r0, c0 = R // 3 + 7, C - 1

@@ -152,8 +152,8 @@ def test_random_axis_scan(device, oracle, shape, strides, offset, axis, dtype, o
 def _narrow_cases(seed, count, scan):
     """Axis 0 of dense row-major matrices with 2 to 255 columns and more
     than 1024 rows, at element offsets 0-4: the period-form sums (up to 95
-    columns), the column tiles beyond, and the row-tile scans (one pass up
-    to 24 columns, three beyond)."""
+    columns), the column tiles beyond, and the scans in row tiles (up to 24
+    columns) and strips."""
     rng = np.random.default_rng(seed)
     out = []
     for i in range(count):
@@ -196,7 +196,7 @@ def test_case_lists_cover_the_layouts_and_paths():
         assert any(c[0][1] <= 8 for c in cases) and any(c[0][0] > 4096 for c in cases)
         assert all(c[0][0] * c[0][1] <= (1 << 21) for c in cases)
     # The narrow sweeps reach each form: period sums (<= 95 columns) and
-    # column tiles, one-pass (<= 24) and three-pass row-tile scans.
+    # column tiles, row-tile scans (<= 24) and strips.
     widths = [p.values[0][1] for p in _narrow_cases(13, 40, False)]
     assert any(c <= 95 for c in widths) and any(c >= 96 for c in widths)
     widths = [p.values[0][1] for p in _narrow_cases(14, 40, True)]
