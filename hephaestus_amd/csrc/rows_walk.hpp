@@ -146,7 +146,10 @@ inline RowsGeom rows_geom(const RowsView &v, bool vec, uint64_t step) {
 // 53.5 / 98.6 / 72.6 / 72.4 -> 42.9 / 81.6 / 42.9 / 45.1 (5.5 to 6.4 TB/s of the
 // lines touched); 114 rows of 674 6.4 / 5.8 / 5.6 / 9.3 -> 4.2 / 3.9 / 3.9 / 5.5.
 // Two units in flight: 18.8 / 27.4 / 18.9 / 16.6 for the first; eight 14.5 /
-// 25.9 / 14.8 / 16.3, but 2 to 5% slower beyond 256 MB.
+// 25.9 / 14.8 / 16.3, but 2 to 5% slower beyond 256 MB.  It wins down to rows of
+// one vector and a tail: 2^24 elements in rows of 5 / 9 / 17 / 33, one element
+// apart, sum 27.0 / 24.6 / 23.5 / 21.6 -> 16.5 / 15.6 / 15.1 / 13.9, dot of rows of
+// 5 46.4 -> 28.9.
 //
 // A row's last unit, when cols is no multiple of 4, is the vector that ends
 // at the row's end: its first `shift` elements belong to the unit before and
