@@ -1,8 +1,9 @@
 """Small downloads: sizes around the pinned slots' and a word's, odd addresses,
-results of kernels queued just before, long queues, an error left by an earlier
-call, and more threads than slots."""
+results of kernels queued just before, long queues, a source in pinned host
+memory, an error left by an earlier call, and more threads than slots."""
 from __future__ import annotations
 
+import ctypes
 import threading
 
 import numpy as np
@@ -56,6 +57,20 @@ def test_waits_for_long_queued_work(device):
         assert np.array_equal(tail, want.astype(np.uint32)), k
     x.free()
     y.free()
+
+
+def test_source_in_pinned_host_memory(device):
+    """No slot serves it: the general copy does, as for large downloads."""
+    pinned = ctypes.c_void_p()
+    assert _hip().hipHostMalloc(ctypes.byref(pinned), ctypes.c_size_t(4096), 0) == 0
+    try:
+        words = np.frombuffer((ctypes.c_char * 4096).from_address(pinned.value), np.uint32)
+        words[:] = np.arange(1024)
+        got = np.zeros(100, np.uint32)
+        _ffi.check(_ffi.lib().hx_download(device.handle, pinned.value + 40, 100, got.ctypes.data, 100, 4))
+        assert np.array_equal(got, np.arange(10, 110))
+    finally:
+        _hip().hipHostFree(pinned)
 
 
 def test_an_earlier_error_of_the_thread_is_not_the_downloads(device):
